@@ -297,15 +297,15 @@ size_t vh_sum_rows_scratch_bytes(int64_t rows, int64_t C);
 #define VH_GEMM_K_GE_M 3     /* A[m, k] == 0 for k < m (M == K) */
 
 /* vh_gemm_desc.engine: which kernels carry the product. The default is this
- * library's own matrix-core kernels, chosen by shape (large dense unbatched
- * products: the persistent 256-row-tile kernel; everything else: the tiled
- * kernel, split along K where the output alone cannot fill the chip). TILED
- * forces the tiled kernel (tests of its split-K path); LIBRARY hands the
- * dense unbatched products hipBLASLt supports to it (an A/B reference for
- * benchmarks) and runs the rest as DEFAULT; WIDE is DEFAULT with the
- * persistent kernel's 256 x 256 tile wherever that kernel runs (tests of the
- * tile DEFAULT picks only for long k loops over many tiles). No counterpart
- * in the reference. */
+ * library's own matrix-core kernels, chosen by shape (large dense products: the
+ * persistent 256-row-tile kernel, whose f32 products run as exact three-part
+ * bf16 splits; everything else: the tiled kernel, split along K where the output
+ * alone cannot fill the chip). TILED forces the tiled kernel (tests of its
+ * split-K path); LIBRARY hands the dense unbatched products hipBLASLt supports to
+ * it (an A/B reference for benchmarks) and runs the rest as DEFAULT; WIDE is
+ * DEFAULT with the large dense products on the f32 matrix instruction (the
+ * persistent kernel's 256 x 256 tile): every k rounds into the f32 sum on its own,
+ * in one fixed order. No counterpart in the reference. */
 #define VH_GEMM_ENGINE_DEFAULT 0
 #define VH_GEMM_ENGINE_TILED 1
 #define VH_GEMM_ENGINE_LIBRARY 2
@@ -341,7 +341,7 @@ int vh_gemm(const vh_gemm_desc* d, void* stream);
 #define VH_GEMM_PATH_NONE 0
 #define VH_GEMM_PATH_TILED 1       /* 128-row tiles, one pass over K */
 #define VH_GEMM_PATH_SPLIT_K 2     /* 128-row tiles over K ranges + fixed-order reduce */
-#define VH_GEMM_PATH_PERSISTENT 3  /* persistent 256 x 192 tiles, stream-K last round */
+#define VH_GEMM_PATH_PERSISTENT 3  /* persistent 256-row tiles, stream-K last round */
 #define VH_GEMM_PATH_LIBRARY 4     /* hipBLASLt */
 #define VH_GEMM_PATH_BATCHED 5     /* persistent walk over batched short-K products */
 int vh_gemm_last_path(void);

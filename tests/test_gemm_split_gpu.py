@@ -1,0 +1,142 @@
+"""The split persistent product (kernels/gemm_split.h): f32 operands as three bf16
+parts each, six part products on the bf16 matrix instruction. Sizes where its
+tiles, k tail, last round and k ranges can go wrong, every operand layout, against
+float64; infinities, NaN, values whose bf16 rounding overflows and subnormals, which
+the split cannot carry and the kernel recomputes; and its error against the f32
+instruction's.
+
+Bound: a sum of K products in f32 is within K u sum |a||b| of the exact one in any
+order (u = 2^-24); the split's 12 roundings per 16 k are fewer than K, and the part
+products it leaves out are below 2^-24 |a||b| each, so (K + 2) u sum |a||b| holds."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from parity import dev, fetch, out
+from test_block_ops_gpu import gemm_desc
+
+pytestmark = pytest.mark.gpu
+
+
+def product(vh, a, b, akc, bkc, off=0, **kw):
+    """vh_gemm of a [M, K] and b [K, N] stored k- or row-contiguous, `off` floats into
+    their buffers; C has a guard row after it that must come back untouched."""
+    M, K = a.shape
+    N = b.shape[1]
+    pad = np.zeros(off, np.float32)
+    A = dev(vh, np.concatenate([pad, (a if akc else a.T).reshape(-1)]))
+    B = dev(vh, np.concatenate([pad, (b.T if bkc else b).reshape(-1)]))
+    C = dev(vh, np.full((M + 1, N), 7.0, np.float32))
+    d = gemm_desc(vh, M, N, K, A.ptr + 4 * off, K if akc else 1, 1 if akc else M, B.ptr + 4 * off, 1 if bkc else N,
+                  K if bkc else 1, C.ptr, N, **kw)
+    vh.check(vh.lib.vh_gemm(ctypes.byref(d), None))
+    path = vh.lib.vh_gemm_last_path()
+    got = fetch(vh, C, (M + 1, N))
+    np.testing.assert_array_equal(got[M], 7.0)
+    return got[:M], path
+
+
+LAYOUTS = [(True, True), (True, False), (False, True), (False, False)]
+#   M, N, K, floats off 16-byte alignment
+SIZES = [
+    (256, 192, 1366, 0),    # one tile, k tail of 6, split over all workgroups
+    (257, 193, 1361, 1),    # one row and one column past a tile, k tail of 1
+    (1000, 777, 1007, 3),   # ragged, k tail of 15
+    (4097, 3071, 32, 0),    # 17 x 12 tiles of two k tiles, last round left whole
+    (300, 500, 16385, 0),   # past the single-chain limit: three k ranges, the last ragged
+]
+
+
+@pytest.mark.parametrize("size", SIZES, ids=str)
+@pytest.mark.parametrize("akc,bkc", LAYOUTS)
+def test_split_product_sizes(vh, akc, bkc, size):
+    M, N, K, off = size
+    print("split", size, akc, bkc, flush=True)
+    r = np.random.default_rng(M + N + K)
+    a = r.standard_normal((M, K)).astype(np.float32)
+    b = r.standard_normal((K, N)).astype(np.float32)
+    got, path = product(vh, a, b, akc, bkc, off)
+    assert path == vh.GEMM_PATH_PERSISTENT
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    bound = (K + 2) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))
+    assert np.all(np.abs(got - ref) <= bound)
+    again, _ = product(vh, a, b, akc, bkc, off)
+    np.testing.assert_array_equal(again, got)
+
+
+@pytest.mark.parametrize("akc,bkc", LAYOUTS)
+def test_split_product_special_values(vh, akc, bkc):
+    """Each special value where the f32 instruction (the WIDE engine) puts it; the
+    other elements within the bound of their own exact sums."""
+    print("split specials", akc, bkc, flush=True)
+    M, N, K = 520, 400, 700
+    r = np.random.default_rng(3)
+    a = r.standard_normal((M, K)).astype(np.float32)
+    b = r.standard_normal((K, N)).astype(np.float32)
+    a[5, 17] = np.inf
+    a[6, 699] = -np.inf
+    a[300, 0] = np.nan
+    a[301, 3] = -3.4e38  # finite, infinite as bf16 (one a row: with two, whether a sum overflows is a matter of order)
+    a[302, :] = 0.0
+    a[302, 8] = 3.4e38
+    b[8, 40:60] = 0.0
+    b[100, 70] = np.inf
+    b[101, 71] = np.nan
+    a[400, :] *= np.float32(1e-38)          # parts below bf16's range without the scale
+    a[401, :] *= np.float32(1e-42)          # subnormals
+    a[402, :] *= np.float32(1e30)           # sums past the scaled range
+    b[:, 90] *= np.float32(1e-20)
+    got, path = product(vh, a, b, akc, bkc)
+    assert path == vh.GEMM_PATH_PERSISTENT
+    want, _ = product(vh, a, b, akc, bkc, engine=vh.GEMM_ENGINE_WIDE)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    np.testing.assert_array_equal(got[inf], want[inf])
+    fine = np.isfinite(want)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    with np.errstate(all="ignore"):
+        ref, mag = a64 @ b64, np.abs(a64) @ np.abs(b64)
+    # Sums below the normal range round to 2^-149.
+    bound = (K + 2) * 2.0 ** -24 * mag + K * 2.0 ** -149
+    with np.errstate(all="ignore"):
+        bad = np.argwhere(fine & ~(np.abs(got - ref) <= bound))
+    assert not len(bad), [(i, j, got[i, j], want[i, j], ref[i, j], bound[i, j]) for i, j in bad[:5]]
+
+
+def test_split_product_broadcast_operand(vh):
+    """An operand repeated along k (stride 0) and a k tail: nothing read past K counts."""
+    M, N, K = 300, 260, 1001
+    r = np.random.default_rng(9)
+    col = r.standard_normal(M).astype(np.float32)
+    b = r.standard_normal((K, N)).astype(np.float32)
+    A, B, C = dev(vh, col), dev(vh, b), out(vh, (M, N))
+    d = gemm_desc(vh, M, N, K, A.ptr, 1, 0, B.ptr, N, 1, C.ptr, N)
+    vh.check(vh.lib.vh_gemm(ctypes.byref(d), None))
+    assert vh.lib.vh_gemm_last_path() == vh.GEMM_PATH_PERSISTENT
+    got = fetch(vh, C, (M, N))
+    ref = col[:, None].astype(np.float64) * b.astype(np.float64).sum(0)
+    bound = (K + 2) * 2.0 ** -24 * np.abs(col)[:, None] * np.abs(b).astype(np.float64).sum(0)
+    assert np.all(np.abs(got - ref) <= bound)
+
+
+@pytest.mark.parametrize("K,one_signed", [(768, False), (3072, False), (16384, False), (16384, True)])
+def test_split_product_error_is_no_larger(vh, K, one_signed):
+    """2-norm error against float64 beside the f32 instruction's (the WIDE engine):
+    of the elements no larger (1.05 for the draw), of their sums over 512 rows and 768
+    columns within 3 times (a bias that all elements share would make it 16 to 28)."""
+    M, N = 512, 768
+    r = np.random.default_rng(K)
+    a = r.standard_normal((M, K)).astype(np.float32)
+    b = r.standard_normal((K, N)).astype(np.float32)
+    if one_signed:
+        a, b = np.abs(a), np.abs(b)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+
+    def errors(engine):
+        d = product(vh, a, b, True, True, engine=engine)[0] - ref
+        return [np.linalg.norm(x) for x in (d, d.sum(0), d.sum(1))]
+    split, f32 = errors(vh.GEMM_ENGINE_DEFAULT), errors(vh.GEMM_ENGINE_WIDE)
+    print("split errors", K, one_signed, split, f32, flush=True)
+    assert split[0] <= 1.05 * f32[0]
+    assert split[1] <= 3 * f32[1] and split[2] <= 3 * f32[2]  # (no drift common to a row or a column)

@@ -244,9 +244,13 @@ struct vb_gpt {
       VB(vh_gemm(&d, nullptr));
     }
     // dW = dlogits^T lnf straight into the gradient's [Vp, D] layout: A is
-    // dlogits read row-contiguous (m-contiguous), B is lnf; the large-product
-    // kernel's wide tile runs it at 8.93 ms, against 8.92 ms for the
-    // transposed product plus ~100 us of transposing copies on either side.
+    // dlogits read row-contiguous (m-contiguous), B is lnf. It stays on the f32
+    // instruction (8.85 ms; the split kernel runs it in 5.6): in the rows of
+    // frequent tokens a sum of ~16384 terms holds a few large ones (-1 / R x per
+    // hit) and many of 1e-5 that size, which one rounding per k loses under the
+    // sum and the split's rounding per eight products does not -- 7.7e-5 against
+    // 5.4e-6 of the gradient's norm from the 64-bit one, so the two kernels'
+    // results differ by 6e-5, more than this gradient may change by.
     {
       vh_gemm_desc d{};
       d.M = Vp;
@@ -262,7 +266,7 @@ struct vb_gpt {
       d.c_sm = D;
       d.batch[0] = d.batch[1] = 1;
       d.alpha = 1.0f;
-      d.engine = engine;
+      d.engine = engine == VH_GEMM_ENGINE_DEFAULT ? VH_GEMM_ENGINE_WIDE : engine;
       VB(vh_gemm(&d, nullptr));
     }
     VB(vh_layernorm_bwd(h2, p(18), dlnf, dh, gr(18), gr(19), R, D, kEps, nullptr, 0, nullptr));

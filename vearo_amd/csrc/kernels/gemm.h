@@ -31,6 +31,7 @@
 //   3: only k >= m contributes (P^T dO and dS^T Q).
 #pragma once
 #include "common.h"
+#include "split3.h"
 
 #define GM_TM VH_GEMM_TILE_M
 #define GM_TK 32
@@ -38,8 +39,6 @@
 #define GM_LT (GM_TM + 4)  // [k][row] LDS stride (floats)
 #define GM_STAGE (GM_TM * GM_LS > GM_TK * GM_LT ? GM_TM * GM_LS : GM_TK * GM_LT)  // one 128-row operand tile
 #define GM_GROUP 8         // tile rows per group in the launch order (L2 reuse of B)
-
-typedef float vh_f32x16 __attribute__((ext_vector_type(16)));
 
 template <bool B>
 struct GmFlag {

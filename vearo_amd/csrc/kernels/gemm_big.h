@@ -585,13 +585,13 @@ VH_DEV void gemm_big_impl(const GemmArgs& a) {
 
 // Finishes the tiles of the stream-K round that were split between
 // workgroups: C = epilogue(sum of the pieces in k order). Workgroup
-// (blockIdx.x) takes 16 rows of split tile blockIdx.x / (256 / 16).
-template <int BN>
+// (blockIdx.x) takes a.fix_rows rows of split tile blockIdx.x / (256 / a.fix_rows).
+template <int BN, class Split>
 VH_DEV void gemm_big_fix_impl(const GemmArgs& a) {
   const int G = a.ksplit;  // the main kernel's grid
-  const GbSplit sp(a, G);
-  const int t = (int)(blockIdx.x / (GB_TM / 16));
-  const int rows0 = (int)(blockIdx.x % (GB_TM / 16)) * 16;
+  const Split sp(a, G);
+  const int parts = GB_TM / a.fix_rows;
+  const int t = (int)blockIdx.x / parts, rows0 = (int)blockIdx.x % parts * a.fix_rows;
   if (t >= sp.rem) return;
   // Workgroups whose runs meet tile t: [glo, ghi].
   const int lo = t * sp.nk, hi = lo + sp.nk;
@@ -619,7 +619,7 @@ VH_DEV void gemm_big_fix_impl(const GemmArgs& a) {
   const float* const Eb = a.E ? a.E + sg.eo : nullptr;
   const int64_t m0 = (int64_t)tm * GB_TM, n0 = (int64_t)tn * BN;
   constexpr int Q = BN / 4;  // 128-bit pieces per row
-  for (int f = threadIdx.x; f < 16 * Q; f += 256) {
+  for (int f = threadIdx.x; f < a.fix_rows * Q; f += 256) {
     const int rl = rows0 + f / Q, cl = (f % Q) * 4;
     vh_f4 v = {0.0f, 0.0f, 0.0f, 0.0f};
     // The pieces of workgroups glo..ghi, four at a time: the four loads go

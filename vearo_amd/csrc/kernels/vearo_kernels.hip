@@ -10,6 +10,7 @@
 #include "gelu.h"
 #include "gemm.h"
 #include "gemm_big.h"
+#include "gemm_split.h"
 #include "generic.h"
 #include "layernorm.h"
 #include "optim.h"
@@ -252,10 +253,9 @@ K_GEMMP(false, false, vh_gemmp_m4_n4)
 
 extern "C" __global__ void __launch_bounds__(256) vh_gemm_reduce(GemmReduceArgs a) { gemm_reduce_impl(a); }
 
-// Large dense products: vh_gemmb_<A><B>_<BN>, persistent 256 x BN tiles (one
-// 512-thread workgroup per CU), and the fix-up of its stream-K round. BN = 256
-// for long k loops over a row-contiguous B (the lm_head dW products), 192
-// otherwise.
+// Large dense products on the f32 instruction: vh_gemmb_<A><B>_<BN>, persistent
+// 256 x BN tiles (one 512-thread workgroup per CU), and the fix-up of its
+// stream-K round.
 #define K_GEMMB(AK, BK, BN, NAME) \
   extern "C" __global__ void __launch_bounds__(512, 1) NAME(GemmArgs a) { gemm_big_impl<AK, BK, BN, 8>(a); }
 K_GEMMB(true, true, 192, vh_gemmb_kk_192)
@@ -266,8 +266,22 @@ K_GEMMB(true, true, 256, vh_gemmb_kk_256)
 K_GEMMB(true, false, 256, vh_gemmb_kn_256)
 K_GEMMB(false, true, 256, vh_gemmb_mk_256)
 K_GEMMB(false, false, 256, vh_gemmb_mn_256)
-extern "C" __global__ void __launch_bounds__(256) vh_gemmb_fix_192(GemmArgs a) { gemm_big_fix_impl<192>(a); }
-extern "C" __global__ void __launch_bounds__(256) vh_gemmb_fix_256(GemmArgs a) { gemm_big_fix_impl<256>(a); }
+extern "C" __global__ void __launch_bounds__(256) vh_gemmb_fix_192(GemmArgs a) { gemm_big_fix_impl<192, GbSplit>(a); }
+extern "C" __global__ void __launch_bounds__(256) vh_gemmb_fix_256(GemmArgs a) { gemm_big_fix_impl<256, GbSplit>(a); }
+
+// The same on the bf16 instruction, operands split in three parts.
+#define K_GEMMS(AK, BK, BN, NAME) \
+  extern "C" __global__ void __launch_bounds__(512, 1) NAME(GemmArgs a) { gemm_split_impl<AK, BK, BN>(a); }
+K_GEMMS(true, true, 192, vh_gemms_kk_192)
+K_GEMMS(true, false, 192, vh_gemms_kn_192)
+K_GEMMS(false, true, 192, vh_gemms_mk_192)
+K_GEMMS(false, false, 192, vh_gemms_mn_192)
+K_GEMMS(true, true, 256, vh_gemms_kk_256)
+K_GEMMS(true, false, 256, vh_gemms_kn_256)
+K_GEMMS(false, true, 256, vh_gemms_mk_256)
+K_GEMMS(false, false, 256, vh_gemms_mn_256)
+extern "C" __global__ void __launch_bounds__(256) vh_gemms_fix_192(GemmArgs a) { gemm_big_fix_impl<192, GsSplit>(a); }
+extern "C" __global__ void __launch_bounds__(256) vh_gemms_fix_256(GemmArgs a) { gemm_big_fix_impl<256, GsSplit>(a); }
 
 // AdamW
 extern "C" __global__ void __launch_bounds__(256) vh_adamw_v1(AdamArgs a) { adamw_impl<1>(a); }

@@ -1459,46 +1459,126 @@ GemmArgs gemm_args(const vh_gemm_desc* d, int64_t lda, int64_t ldb, int64_t tile
 namespace {
 thread_local int g_gemm_path = VH_GEMM_PATH_NONE;
 
-// The persistent 256 x BN-tile kernel (kernels/gemm_big.h) for a large dense
-// product, when its conditions hold; *taken reports whether it ran. BN = 256
-// when B is row-contiguous, the k loop is long (K >= VH_GEMMB_WIDE_K) and the
-// wide tiles fill at least one round of workgroups: a wider tile does a third
-// more products per k-tile barrier and loads 14 % fewer operand bytes per
-// product (on MI355X, the lm_head dW as [50260, 768] 9.16 -> 8.93 ms, as
-// [768, 50260] 9.07 -> 8.92), while its epilogue keeps fewer registers free
-// (it spills), which short k loops pay for (fc2 forward, K = 3072: 544 -> 593
-// us), and a product of fewer wide tiles than workgroups runs all of them in
-// the stream-K round (the [768, 768] weight gradient, K = 16384: 180 -> 196
-// us). With both operands k-contiguous the narrow tile stays ahead even on
-// long k loops (lm_head dx, K = 50260: 8.65 against 9.00 ms).
-// Conditions: 4-byte-aligned operand bases (its 128-bit loads need no more); a
-// tile's reads within 2^32 bytes of its origin (leading dimensions < 2^22); k
-// tile and tile counts below 2^31 (K < 2^26). A k-contiguous operand with
-// K % 32 != 0 splits K: the kernel takes the whole 32-wide k tiles and the
-// tiled kernel adds the rest (alpha times the tail product) into C. A
-// row-contiguous operand's reads past K land past its buffer bound, and so read
-// 0, only when its leading dimension covers its extent (lda >= M, ldb >= N):
-// one broadcast along k (stride 0) or with overlapping rows leaves a partial
-// last k tile to the tiled kernel, which tests k < K.
+// How the persistent kernel (kernels/gemm_split.h) runs a product: tile width and
+// whether the last, partly filled round of tiles is split along K over all
+// workgroups (stream-K) or run as it is on as many workgroups as it has tiles.
+struct SplitPlan {
+  int64_t bn;
+  bool whole_tail;
+  double us;  // the estimate the choice was made by
+};
+
+// Estimated time of each form. The kernel is bound by the chip's power, not by
+// its clock limit: measured on MI355X, a k step takes 2.40 us (256 wide) or 1.82
+// us (192 wide: 1 % more per column) with all 256 workgroups busy, in proportion
+// to how many are, but no less than 1.4 / 1.05 us (2.4 GHz). So an unsplit round
+// on a share f of the chip loses max(1.4 - 2.4 f, 0.09) us per k tile, while a
+// split one writes and reads back a 256 KB (192 KB) piece per workgroup and tile,
+// ~0.1 us each, plus the fix-up's launch. Measured, 256 / 192 wide: N = 50272 over
+// K = 768 5.71 / 5.99 ms; N = 3072 345 / 364 us; N = 2304 (2.25 / 3 rounds) 286 / 273; N =
+// 768 (192 / 256 tiles): K = 768 99 / 94, K = 3072 367 / 349 us, K = 50272 5.82 /
+// 5.63 ms. Split / unsplit at 256 wide: 192 tiles of 48 k tiles 138 / 99 us, of 192
+// 388 / 363, of 3142 5.81 / 6.01 ms; 64 tiles of 48 296 / 310 us; 9 of 1024 118 / 1640.
+SplitPlan gemm_split_plan(int64_t M, int64_t N, int64_t K, int64_t nb, int G) {
+  SplitPlan best{0, false, 0.0};
+  const double nk = (double)cdiv(K, VH_GEMMS_TK);
+  for (int64_t bn : {VH_GEMMB_TN_WIDE, VH_GEMMB_TN}) {
+    const double share = bn == VH_GEMMB_TN_WIDE ? 1.0 : 0.75, step = bn == VH_GEMMB_TN_WIDE ? 2.40 : 1.82;
+    const int64_t tiles = cdiv(M, VH_GEMMB_TM) * cdiv(N, bn) * nb, rem = tiles % G;
+    const double whole = nk * std::max(1.4 * share - step * (double)rem / G, 0.09 * share);
+    const double split = 5.0 + 0.1 * share * (double)(G + rem);
+    const double us = nk * step * (double)tiles / G + (rem ? std::min(whole, split) : 0.0);
+    if (!best.bn || us < best.us) best = SplitPlan{bn, rem > 0 && whole < split, us};
+  }
+  return best;
+}
+
+// Whether the persistent kernels take a product: dense, large, 4-byte-aligned
+// operand bases (their 128-bit loads need no more), a tile's reads within 2^32
+// bytes of its origin (leading dimensions < 2^22), k tile and tile counts below
+// 2^31. Batched products need k loops long enough for a persistent walk (short-K
+// batched products, such as attention's scores, have their own kernel).
+bool gemm_persistent_ok(const vh_gemm_desc* d, int64_t lda, int64_t ldb) {
+  const int64_t M = d->M, N = d->N, K = d->K, nb = d->batch[0] * d->batch[1];
+  return d->causal == VH_GEMM_DENSE && K > 0 && (nb == 1 || K >= 512) && M >= VH_GEMMB_TM && N >= VH_GEMMB_TN &&
+         (double)M * (double)N * (double)K * (double)nb >= 67108864.0 &&
+         reinterpret_cast<uintptr_t>(d->a) % 4 == 0 && reinterpret_cast<uintptr_t>(d->b) % 4 == 0 &&
+         lda < (int64_t(1) << 22) && ldb < (int64_t(1) << 22) && K < (int64_t(1) << 26) &&
+         (double)cdiv(M, VH_GEMMB_TM) * (double)cdiv(N, VH_GEMMB_TN) * (double)nb < (double)INT32_MAX;
+}
+
+// One launch of the split persistent kernel (and its fix-up).
+int gemm_split_range(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t ldb, hipStream_t s) {
+  const int64_t M = d->M, N = d->N, K = d->K, nb = d->batch[0] * d->batch[1];
+  const int G = std::max(8, g_rt.cu_count / 8 * 8);
+  const SplitPlan plan = gemm_split_plan(M, N, K, nb, G);
+  const int64_t tiles_m = cdiv(M, VH_GEMMB_TM), tiles_n = cdiv(N, plan.bn), rem = tiles_m * tiles_n * nb % G;
+  GemmArgs g = gemm_args(d, lda, ldb, tiles_m, tiles_n);
+  g.nbat = nb;
+  g.whole_tail = plan.whole_tail ? 1 : 0;
+  void* ws = nullptr;
+  if (rem > 0 && !plan.whole_tail) {
+    VH_TRY(g_arena.alloc((size_t)(G * VH_GEMMB_SLOTS * VH_GEMMB_TM * plan.bn) * sizeof(float), s, &ws));
+    g.ws = static_cast<float*>(ws);
+  }
+  const std::string bn = std::to_string(plan.bn);
+  int rc = launch(std::string("vh_gemms_") + (akc ? "k" : "m") + (bkc ? "k" : "n") + "_" + bn, G, 1, 512, 0, s, g);
+  if (rc == VH_OK && ws) {
+    GemmArgs x = g;
+    x.ksplit = G;
+    // 16 rows per workgroup, or 4 where that leaves the chip short of
+    // workgroups (9 split tiles: the product 137 -> 118 us; 192: 168 against 138).
+    x.fix_rows = rem * 16 >= 2 * G ? 16 : 4;
+    rc = launch("vh_gemms_fix_" + bn, rem * (VH_GEMMB_TM / x.fix_rows), 1, 256, 0, s, x);
+  }
+  if (ws) g_arena.free(ws, s);
+  return rc;
+}
+
+// A large dense product on the split persistent kernel. A chain over very long
+// K loses small part products under a sum they no longer move, alike in every
+// row that shares a large term (the lm_head dx of the GPT step over K = 50272:
+// column sums over the tokens 7.6e-7 off, against 5.5e-7 on the f32 instruction,
+// though the elements themselves are 2.4e-6 against 5.5e-6). Past 16384 it runs
+// in equal ranges of at most 8192, each accumulating into C (2 M N floats of
+// traffic per range).
+int gemm_split(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t ldb, hipStream_t s, bool* taken) {
+  *taken = false;
+  if (!gemm_persistent_ok(d, lda, ldb)) return VH_OK;
+  const int64_t K = d->K, n = K > 16384 ? cdiv(K, 8192) : 1;
+  const int64_t kc = cdiv(cdiv(K, n), VH_GEMMS_TK) * VH_GEMMS_TK;
+  for (int64_t k0 = 0; k0 < K; k0 += kc) {
+    vh_gemm_desc t = *d;
+    t.K = std::min(kc, K - k0);
+    t.a = d->a + k0 * d->a_sk;
+    t.b = d->b + k0 * d->b_sk;
+    if (k0 > 0) {
+      t.e = nullptr;
+      t.accumulate = 1;
+    }
+    VH_TRY(gemm_split_range(&t, akc, bkc, lda, ldb, s));
+  }
+  *taken = true;
+  g_gemm_path = VH_GEMM_PATH_PERSISTENT;
+  return VH_OK;
+}
+
+// The f32-instruction persistent kernel (kernels/gemm_big.h) with its 256 x 256
+// tile (256 x 192 below 256 columns), for the WIDE engine. A k-contiguous operand with K % 32 != 0 splits K: the
+// kernel takes the whole 32-wide k tiles and the tiled kernel adds the rest
+// (alpha times the tail product) into C. A row-contiguous operand's reads past K
+// land past its buffer bound, and so read 0, only when its leading dimension
+// covers its extent (lda >= M, ldb >= N): one broadcast along k (stride 0) or with
+// overlapping rows leaves a partial last k tile to the tiled kernel.
 int gemm_big(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t ldb, hipStream_t s, bool* taken) {
   *taken = false;
   const int64_t M = d->M, N = d->N, K = d->K, nb = d->batch[0] * d->batch[1];
-  if (d->causal != VH_GEMM_DENSE || K <= 0) return VH_OK;
-  // Batched products need k loops long enough for a persistent walk (short-K
-  // batched products, such as attention's scores, have their own kernel).
-  if (nb > 1 && K < 512) return VH_OK;
-  if (M < VH_GEMMB_TM || N < VH_GEMMB_TN || (double)M * (double)N * (double)K * (double)nb < 67108864.0)
-    return VH_OK;
-  if (reinterpret_cast<uintptr_t>(d->a) % 4 != 0 || reinterpret_cast<uintptr_t>(d->b) % 4 != 0) return VH_OK;
-  if (lda >= (int64_t(1) << 22) || ldb >= (int64_t(1) << 22) || K >= (int64_t(1) << 26)) return VH_OK;
+  if (!gemm_persistent_ok(d, lda, ldb)) return VH_OK;
   const int G = std::max(8, g_rt.cu_count / 8 * 8);
   const int64_t K32 = (akc || bkc) ? K / 32 * 32 : K;
   if (K32 == 0) return VH_OK;
   if (K32 % 32 != 0 && ((!akc && lda < M) || (!bkc && ldb < N))) return VH_OK;
-  const bool wide = (d->engine == VH_GEMM_ENGINE_WIDE && N >= VH_GEMMB_TN_WIDE) ||
-                    (!bkc && K32 >= VH_GEMMB_WIDE_K && N >= VH_GEMMB_TN_WIDE &&
-                     cdiv(M, VH_GEMMB_TM) * cdiv(N, VH_GEMMB_TN_WIDE) * nb >= G);
-  const int64_t BN = wide ? VH_GEMMB_TN_WIDE : VH_GEMMB_TN;
+  const int64_t BN = N >= VH_GEMMB_TN_WIDE ? VH_GEMMB_TN_WIDE : VH_GEMMB_TN;
   const int64_t tiles_m = cdiv(M, VH_GEMMB_TM), tiles_n = cdiv(N, BN);
   if (tiles_m * tiles_n * nb >= INT32_MAX) return VH_OK;
   const int64_t tiles = tiles_m * tiles_n * nb, rem = tiles % G;
@@ -1516,6 +1596,7 @@ int gemm_big(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t ldb
   if (rc == VH_OK && rem > 0) {
     GemmArgs f = g;
     f.ksplit = G;
+    f.fix_rows = 16;
     rc = launch("vh_gemmb_fix_" + bn, (rem * (VH_GEMMB_TM / 16)), 1, 256, 0, s, f);
   }
   if (ws) g_arena.free(ws, s);
@@ -1584,7 +1665,7 @@ int vh_gemm(const vh_gemm_desc* d, void* stream) {
   }
   if (!dflag && d->engine != VH_GEMM_ENGINE_TILED) {
     bool taken = false;
-    VH_TRY(gemm_big(d, akc, bkc, lda, ldb, S(stream), &taken));
+    VH_TRY((d->engine == VH_GEMM_ENGINE_WIDE ? gemm_big : gemm_split)(d, akc, bkc, lda, ldb, S(stream), &taken));
     if (taken) return VH_OK;
   }
   const bool avec = K > 0 && gemm_vec_ok(d->a, lda, akc ? K : M, d->a_sb);

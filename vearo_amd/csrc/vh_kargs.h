@@ -96,12 +96,13 @@ struct SoftmaxArgs {
 // C tile of one GEMM workgroup (host and device agree on the grid).
 #define VH_GEMM_TILE_M 128
 #define VH_GEMM_TILE_N 128
-// The persistent kernel for large dense products (kernels/gemm_big.h): C tile
-// rows x columns, and the workspace slots per workgroup of its stream-K round.
+// The persistent kernels for large dense products (kernels/gemm_split.h, and on
+// the f32 instruction kernels/gemm_big.h): C tile rows x columns, and the
+// workspace slots per workgroup of their stream-K round.
 #define VH_GEMMB_TM 256
-#define VH_GEMMB_TN 192       // the default tile width (and the smallest N it takes)
-#define VH_GEMMB_TN_WIDE 256  // the tile width for long k loops over a row-contiguous B
-#define VH_GEMMB_WIDE_K 8192  // K (whole k tiles) from which the wide tile is used
+#define VH_GEMMB_TN 192       // the narrow tile (and the smallest N they take)
+#define VH_GEMMB_TN_WIDE 256
+#define VH_GEMMS_TK 16        // gemm_split's k tile
 #define VH_GEMMB_SLOTS 2
 
 struct GemmArgs {
@@ -127,6 +128,8 @@ struct GemmArgs {
   float* ws;
   int64_t nbat;  // persistent form (vh_gemmp_*): batches in the launch (grid y is 1)
   const int32_t* causal_flag;  // non-null: `causal` applies only when *causal_flag is 1, else dense
+  int32_t whole_tail;          // vh_gemms_*: 1 leaves the last round's tiles unsplit
+  int32_t fix_rows;            // vh_gemm[bs]_fix_*: tile rows per workgroup (divides 256)
 };
 
 // Fixed-order sum of the split-K partials plus the GEMM epilogue.
