@@ -339,9 +339,9 @@ int vh_gemm(const vh_gemm_desc* d, void* stream);
  * VH_GEMM_PATH_* (0 before any call, or for an empty product). A diagnostic
  * for tests and benchmarks, no counterpart in the reference. */
 #define VH_GEMM_PATH_NONE 0
-#define VH_GEMM_PATH_TILED 1       /* 128-row tiles, one pass over K */
-#define VH_GEMM_PATH_SPLIT_K 2     /* 128-row tiles over K ranges + fixed-order reduce */
-#define VH_GEMM_PATH_PERSISTENT 3  /* persistent 256-row tiles, stream-K last round */
+#define VH_GEMM_PATH_TILED 1       /* 128- or 64-row tiles, one pass over K */
+#define VH_GEMM_PATH_SPLIT_K 2     /* the same over K ranges + fixed-order reduce */
+#define VH_GEMM_PATH_PERSISTENT 3  /* persistent tiles: 256-row, stream-K last round, or 64 x 64 for the smaller ones */
 #define VH_GEMM_PATH_LIBRARY 4     /* hipBLASLt */
 #define VH_GEMM_PATH_BATCHED 5     /* persistent walk over batched short-K products */
 int vh_gemm_last_path(void);

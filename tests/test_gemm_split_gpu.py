@@ -140,3 +140,66 @@ def test_split_product_error_is_no_larger(vh, K, one_signed):
     print("split errors", K, one_signed, split, f32, flush=True)
     assert split[0] <= 1.05 * f32[0]
     assert split[1] <= 3 * f32[1] and split[2] <= 3 * f32[2]  # (no drift common to a row or a column)
+
+
+# ------------------------------------------------ the tiled kernel (kernels/gemm.h) --
+
+#   M, N, K, floats off alignment: K <= 8 on the f32 instruction, then edges of its 64 x
+#   64 and 128 x 128 tiles and of its 32-wide k tiles, one and several of each.
+TILE_SIZES = [(64, 64, 1, 0), (65, 63, 8, 1), (63, 65, 9, 0), (1, 200, 33, 3), (200, 1, 31, 0), (129, 127, 95, 2),
+              (64, 128, 32, 0), (700, 130, 65, 1), (255, 300, 2049, 1), (2048, 191, 100, 0)]
+
+
+@pytest.mark.parametrize("size", TILE_SIZES, ids=str)
+@pytest.mark.parametrize("akc,bkc", LAYOUTS)
+def test_tiled_product_sizes(vh, akc, bkc, size):
+    M, N, K, off = size
+    print("tiled", size, akc, bkc, flush=True)
+    r = np.random.default_rng(M + N + K)
+    a = r.standard_normal((M, K)).astype(np.float32)
+    b = r.standard_normal((K, N)).astype(np.float32)
+    got, path = product(vh, a, b, akc, bkc, off)
+    assert path in (vh.GEMM_PATH_TILED, vh.GEMM_PATH_SPLIT_K)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    u = 2.0 ** -24  # (the f32 bound; the split's own two u per product only past K = 8)
+    bound = (K * u / (1 - K * u)) * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))
+    assert np.all(np.abs(got - ref) <= bound)
+
+
+def test_tiled_product_special_values(vh):
+    M, N, K = 150, 140, 70
+    r = np.random.default_rng(4)
+    a = r.standard_normal((M, K)).astype(np.float32)
+    b = r.standard_normal((K, N)).astype(np.float32)
+    a[5, 17], a[6, 69], a[100, 0], a[101, 3] = np.inf, -np.inf, np.nan, 3.4e38
+    a[102, :] = 0.0
+    b[40, 70], b[41, 71] = np.inf, np.nan
+    b[3, 70] = 0.0  # (row 101's term overflows in f32 and not in float64: none beside an infinity)
+    a[120, :] *= np.float32(1e-42)
+    got, _ = product(vh, a, b, True, False)
+    with np.errstate(all="ignore"):
+        a64, b64 = a.astype(np.float64), b.astype(np.float64)
+        want = (a64 @ b64).astype(np.float32)  # one overflowing term a row: its sign is the sum's
+        bound = (K + 2) * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64)) + K * 2.0 ** -149
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+        near = np.abs(want) > 3.39e38  # f32's edge: the sum may or may not round to infinity
+        np.testing.assert_array_equal(got[np.isinf(want) & ~near], want[np.isinf(want) & ~near])
+        fine = np.isfinite(want) & ~near
+        assert np.all(np.isfinite(got[fine])) and np.all(np.abs(got - want)[fine] <= bound[fine] * 1.01)
+
+
+@pytest.mark.parametrize("akc", [True, False])
+def test_tiled_product_far_apart_rows(vh, akc):
+    """A leading dimension past the buffer loads' 32-bit offsets: element by element."""
+    M, K, N, ld = (3, 40, 70, (1 << 22) + 1) if akc else (40, 3, 70, (1 << 22) + 1)
+    r = np.random.default_rng(6)
+    a = r.standard_normal((M, K)).astype(np.float32)
+    b = r.standard_normal((K, N)).astype(np.float32)
+    big = np.zeros((3, ld), np.float32)
+    big[:, :40] = a if akc else a.T
+    A, B, C = dev(vh, big), dev(vh, b), out(vh, (M, N))
+    d = gemm_desc(vh, M, N, K, A.ptr, ld if akc else 1, 1 if akc else ld, B.ptr, N, 1, C.ptr, N)
+    vh.check(vh.lib.vh_gemm(ctypes.byref(d), None))
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    bound = (K + 2) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))
+    assert np.all(np.abs(fetch(vh, C, (M, N)) - ref) <= bound)

@@ -162,27 +162,32 @@ VH_DEV float gm_finish(const GemmArgs& a, const float* E, bool raw, float v, int
   return v;
 }
 
-// A wave's 64 x TN/2 quadrant of the tile at (m0, n0) straight from its
-// accumulators: register r of a 32 x 32 tile holds row 8*(r/4) + 4*h + r%4,
+// A wave's MT x NTW matrix-core tiles of the T-row tile at (m0, n0) straight from
+// its accumulators: register r of a 32 x 32 tile holds row 8*(r/4) + 4*h + r%4,
 // column li; elements outside M x N are dropped. NT: streaming (nontemporal)
 // stores, which do not allocate the written lines in L2.
-template <int NTW, bool NT = false>
-VH_DEV void gm_store_direct(const GemmArgs& a, const vh_f32x16 (&acc)[2][NTW], float* out, int64_t ldo,
-                            const float* E, bool raw, int64_t m0, int64_t n0, int wm, int wn, int li, int h) {
-  if (m0 + GM_TM <= a.M && n0 + NTW * 64 <= a.N && !E && (raw || !a.accumulate)) {
-    // A whole tile that reads nothing back: the stores go out back to back
-    // (a conditional load of C among them makes each wait for all earlier
+template <int MT, int NTW, bool NT = false>
+VH_DEV void gm_store_direct(const GemmArgs& a, const vh_f32x16 (&acc)[MT][NTW], float* out, int64_t ldo,
+                            const float* E, bool raw, int64_t m0, int64_t n0, int T, int wm, int wn, int li, int h) {
+  if (m0 + T <= a.M && n0 + NTW * 64 <= a.N && (raw || !a.accumulate) && (raw || !E || a.sem == 0)) {
+    // A whole tile that reads nothing back but a bias row: the stores go out back
+    // to back (a conditional load of C among them makes each wait for all earlier
     // stores, as the memory counter covers both).
     const float alpha = raw ? 1.0f : a.alpha;
-    float* base = out + (m0 + wm * 64 + 4 * h) * ldo + n0 + wn * (NTW * 32) + li;
+    const bool bias = !raw && E;
+    float* base = out + (m0 + wm * (MT * 32) + 4 * h) * ldo + n0 + wn * (NTW * 32) + li;
+    float eb[NTW];
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+    for (int nt = 0; nt < NTW; ++nt) eb[nt] = bias ? E[(n0 + wn * (NTW * 32) + nt * 32 + li) * a.sen] : 0.0f;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int nt = 0; nt < NTW; ++nt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           float* cp = base + (mt * 32 + 8 * (r >> 2) + (r & 3)) * ldo + nt * 32;
-          const float v = raw ? acc[mt][nt][r] : acc[mt][nt][r] * alpha;
+          float v = raw ? acc[mt][nt][r] : acc[mt][nt][r] * alpha;
+          if (bias) v = v + eb[nt];
           if constexpr (NT)
             __builtin_nontemporal_store(v, cp);
           else
@@ -191,16 +196,23 @@ VH_DEV void gm_store_direct(const GemmArgs& a, const vh_f32x16 (&acc)[2][NTW], f
     return;
   }
 #pragma unroll
-  for (int mt = 0; mt < 2; ++mt) {
+  for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
     for (int nt = 0; nt < NTW; ++nt) {
       const int64_t n = n0 + wn * (NTW * 32) + nt * 32 + li;
+      // (the old C of a whole column goes out before its stores, see above)
+      float old[16];
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int64_t m = m0 + wm * 64 + mt * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+        const int64_t m = m0 + wm * (MT * 32) + mt * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+        old[r] = a.accumulate && !raw && m < a.M && n < a.N ? out[m * ldo + n] : 0.0f;
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int64_t m = m0 + wm * (MT * 32) + mt * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
         if (m < a.M && n < a.N) {
           float* cp = out + m * ldo + n;
-          const float v = gm_finish(a, E, raw, acc[mt][nt][r], m, n, a.accumulate && !raw ? *cp : 0.0f);
+          const float v = gm_finish(a, E, raw, acc[mt][nt][r], m, n, old[r]);
           if constexpr (NT)
             __builtin_nontemporal_store(v, cp);
           else
@@ -211,15 +223,52 @@ VH_DEV void gm_store_direct(const GemmArgs& a, const vh_f32x16 (&acc)[2][NTW], f
   }
 }
 
-template <bool A_KC, bool A_VEC, bool B_KC, bool B_VEC, int TN>
-VH_DEV void gemm_f32_impl(const GemmArgs& a) {
-  static_assert(TN == 128 || TN == 64, "C tile width");
-  constexpr int NTW = TN / 64;  // 32-wide n tiles per wave
-  // L[0..1]: A's two k stages, L[2..3]: B's; after the k loop, the C tile.
-  __shared__ __attribute__((aligned(16))) float L[4][GM_STAGE];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+// Buffer resource of `bytes` bytes from `org`, clamped to [0, 2^32 - 1], and a
+// 128-bit load through it (4-byte alignment is enough; each dword past the end
+// reads 0 on its own).
+VH_DEV __amdgpu_buffer_rsrc_t gm_rsrc(const float* org, int64_t bytes) {
+  uint32_t hi = (uint32_t)((uint64_t)bytes >> 32), lo = (uint32_t)bytes;
+  asm("" : "+s"(hi), "+s"(lo));  // keeps the compiler from joining the halves into a vector compare
+  const uint32_t nrec = (int32_t)hi < 0 ? 0u : (hi != 0 ? 0xFFFFFFFFu : lo);
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(org), (short)0, (int)nrec, 0x00020000);
+}
+VH_DEV vh_f4 gm_bload(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(vh_f4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+
+// The tiled product on the bf16 instruction (split3.h): a 256-thread workgroup
+// computes a T x T tile of C (T = 128 or 64), its four waves T/2 x T/2 quadrants as
+// NW x NW matrix-core tiles of 32 x 32. K advances in tiles of 32: each thread
+// brings T/64 pieces of eight consecutive k of a row of each operand (gt_load),
+// splits them and writes the parts' 16-byte fragments to LDS, laid out [part][k
+// eighth][row]. A k tile's products are summed on their own (tt, 12 roundings of
+// the small sum) and then added to acc in f32, so an element sees one rounding
+// per 32 k at its own size: measured at K = 768, 1.3e-7 of the result against 5.0e-7
+// on the f32 instruction.
+//
+// T = 64 runs two LDS stages, one barrier per k tile, and loads two k tiles ahead:
+// for products whose few tiles leave the chip's latency exposed. T = 128 runs one
+// stage (50 KB, so that two workgroups share a CU and cover each other's barriers
+// and loads) and loads one k tile ahead.
+//
+// BUF operands come through buffer loads, whose bounds make rows past the
+// operand's last element read 0 and which need only 4-byte alignment; the others
+// (leading dimensions whose tile reads pass 2^32 bytes) element by element.
+template <bool A_KC, bool A_BUF, bool B_KC, bool B_BUF, int T>
+struct GemmTile {
+  static constexpr int HS = T * 4 + 16, OP = 12 * HS;  // dwords per k eighth (64 bytes of padding), per operand
+  static constexpr int D = T == 64 ? 2 : 1;            // LDS stages
+  using Lds = uint32_t[D][2][OP];
+  // C tile (tm, tn) of batch `bat`, or its raw partial over K range `kr` of a.ksplit.
+  static VH_DEV void run(const GemmArgs& a, Lds& L, int tm, int tn, int64_t bat, int kr, int causal);
+};
+
+template <bool A_KC, bool A_BUF, bool B_KC, bool B_BUF, int T>
+VH_DEV void gemm_tile_impl(const GemmArgs& a) {
+  using Tile = GemmTile<A_KC, A_BUF, B_KC, B_BUF, T>;
+  __shared__ __attribute__((aligned(1024))) typename Tile::Lds L;
   int tm, tn;
-  int64_t bat = blockIdx.y;  // batch index (both batch dims)
+  int64_t bat = blockIdx.y;  // batch index (both batch dims), or the K range
   const int causal = gm_causal(a);
   if (causal >= 2 && a.ksplit <= 1) {
     // The k range grows with the tile row (k <= m) or shrinks (k >= m): deal
@@ -234,8 +283,34 @@ VH_DEV void gemm_f32_impl(const GemmArgs& a) {
   } else {
     gm_tile_of(blockIdx.x, gridDim.x, a.tiles_m, a.tiles_n, tm, tn);
   }
-  const int64_t m0 = (int64_t)tm * GM_TM, n0 = (int64_t)tn * TN;
-  if (causal == 1 && n0 > m0 + GM_TM - 1) return;  // the whole tile is masked
+  Tile::run(a, L, tm, tn, bat, (int)blockIdx.y, causal);
+}
+
+// The persistent form for dense products: the grid is at most the chip's
+// resident workgroups, each walking the (tile, K range) pairs of all batches.
+template <bool A_KC, bool B_KC, int T>
+VH_DEV void gemm_tile_walk(const GemmArgs& a) {
+  using Tile = GemmTile<A_KC, true, B_KC, true, T>;
+  __shared__ __attribute__((aligned(1024))) typename Tile::Lds L;
+  const int tiles = a.tiles_m * a.tiles_n;
+  const int64_t items = (int64_t)tiles * (a.ksplit > 1 ? a.ksplit : a.nbat);
+  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
+    int tm, tn;
+    gm_tile_of((int)(it % tiles), tiles, a.tiles_m, a.tiles_n, tm, tn);
+    Tile::run(a, L, tm, tn, it / tiles, (int)(it / tiles), 0);
+    __syncthreads();  // the next item stages into the LDS this one read
+  }
+}
+
+template <bool A_KC, bool A_BUF, bool B_KC, bool B_BUF, int T>
+VH_DEV void GemmTile<A_KC, A_BUF, B_KC, B_BUF, T>::run(const GemmArgs& a, Lds& L, int tm, int tn, int64_t bat, int kr,
+                                                       int causal) {
+  static_assert(T == 128 || T == 64, "tile");
+  constexpr int NW = T / 64, U = T / 64;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int wm = w >> 1, wn = w & 1, li = lane & 31, h = lane >> 5, q4 = lane >> 4, c4 = lane & 15;
+  const int64_t m0 = (int64_t)tm * T, n0 = (int64_t)tn * T;
+  if (causal == 1 && n0 > m0 + T - 1) return;  // the whole tile is masked
 
   const bool split = a.ksplit > 1;
   const int64_t b1 = split ? 0 : bat / a.nb2, b2 = split ? 0 : bat % a.nb2;
@@ -244,173 +319,217 @@ VH_DEV void gemm_f32_impl(const GemmArgs& a) {
   float* C = a.C + b1 * a.sc1 + b2 * a.sc2;
 
   int64_t kb = 0, ke = a.K;
-  if (causal == 2) ke = m0 + GM_TM < a.K ? m0 + GM_TM : a.K;
+  if (causal == 2) ke = m0 + T < a.K ? m0 + T : a.K;
   if (causal == 3) kb = (m0 / GM_TK) * GM_TK;
   if (split) {
-    kb = (int64_t)blockIdx.y * a.kchunk;
+    kb = (int64_t)kr * a.kchunk;
     ke = kb + a.kchunk < a.K ? kb + a.kchunk : a.K;
   }
+  // K <= 8 runs on the f32 instruction (below): a single product there is correctly
+  // rounded, the split's is up to 0.94 ulp off (1.9 u, measured over 65536), which
+  // more products' own roundings cover.
+  const bool tiny = a.K <= 8;
+  const int steps = ke > kb && !tiny ? (int)((ke - kb + GM_TK - 1) / GM_TK) : 0;
 
-  vh_f32x16 acc[2][NTW];
+  // Piece u of a thread: row and k eighth, and its dword in an LDS part. k-contiguous:
+  // four threads cover a row's 128 bytes. Row-contiguous: wave w takes 64-row
+  // block (w + 4 u) / 4 and k eighth (w + 4 u) % 4; lane 16 q + c loads rows 4 c .. 4 c + 3
+  // at k = 2 q and 2 q + 1, and a transpose across the lanes' q leaves it all eight k of
+  // row 4 c + q (at LDS piece 16 q + (c + 4 q) % 16 of the block, which the writes and
+  // the fragment reads of 16 lanes both meet without bank conflicts).
+  auto k8_of = [&](bool kc, int u) { return kc ? tid & 3 : (w + 4 * u) & 3; };
+  auto lds_of = [&](bool kc, int u) {
+    const int piece = kc ? (tid >> 2) + 64 * u : ((w + 4 * u) >> 2) * 64 + 16 * q4 + ((c4 + 4 * q4) & 15);
+    return k8_of(kc, u) * HS + 4 * piece;
+  };
+  vh_f4 ra[D][U][2], rb[D][U][2];
+  // The pieces of the k tile at k0 of rows r0 .. (R of them, K long) into v.
+  auto load = [&](auto kcv, auto bufv, const float* X, int64_t ld, int64_t r0, int64_t R, int64_t k0,
+                  vh_f4 (&v)[U][2]) {
+    constexpr bool KC = decltype(kcv)::value, BUF = decltype(bufv)::value;
+    if constexpr (BUF) {
+      const auto r = gm_rsrc(X + (KC ? r0 * ld + k0 : k0 * ld + r0),
+                             (KC ? (R - 1 - r0) * ld + a.K - k0 : (a.K - 1 - k0) * ld + R - r0) * 4);
+      const uint32_t ld4 = (uint32_t)ld * 4u;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < NTW; ++j) acc[i][j] = vh_f32x16{};
-
-  const int wm = w >> 1, wn = w & 1, li = lane & 31, h = lane >> 5;
-  float sa[GM_TM / 8], sb[TN / 8];
-  int s = 0;
-  if (kb < ke) {
-    gm_load<A_KC, A_VEC, GM_TM>(A, a.lda, m0, a.M, kb, a.K, tid, sa);
-    gm_load<B_KC, B_VEC, TN>(B, a.ldb, n0, a.N, kb, a.K, tid, sb);
-    gm_store_lds<A_KC, A_VEC, GM_TM>(L[0], tid, sa);
-    gm_store_lds<B_KC, B_VEC, TN>(L[2], tid, sb);
-    __syncthreads();
-  }
-  // Per k tile: the next tile's global loads go out; then all of this tile's
-  // fragments are read from LDS at once (the products wait only on the reads
-  // they use, which return in order); the next tile is written to the other
-  // LDS buffer (free since the last barrier) between the last group's
-  // products. On the last tile that write goes to a buffer nothing reads again
-  // (the loop body stays one block, so the order below holds).
-  // A tile entirely inside A, B and K (all but the edge tiles) runs a copy of
-  // the loop without bounds tests or branches around its loads; on the last
-  // k tile they fetch that tile again rather than branch.
-  constexpr int RD = 4 * ((A_KC ? 2 : 8) + NTW * (B_KC ? 1 : 4));              // LDS reads per tile
-  constexpr int WR = (A_VEC ? GM_TM / 32 : GM_TM / 8) + (B_VEC ? TN / 32 : TN / 8);  // LDS writes per tile
-  constexpr int VM = (A_VEC ? GM_TM / 32 : GM_TM / 8) + (B_VEC ? TN / 32 : TN / 8);  // global loads per tile
-  constexpr int MF = 8 * NTW;                                                   // products per 4-k group
-  // One k step on the k tile staged in stage sc: the loads of k tile kl go
-  // out into (la, lb), this tile's products run, and (wa, wb) -- the k tile
-  // that follows this one -- are staged into the other LDS buffers.
-  auto kstep = [&](auto unchecked, int sc, float (&la)[GM_TM / 8], float (&lb)[TN / 8],
-                   const float (&wa)[GM_TM / 8], const float (&wb)[TN / 8], int64_t kl, bool load) {
-    constexpr bool CHECK = !decltype(unchecked)::value;
-    if constexpr (CHECK) {
-      if (load) {
-        gm_load<A_KC, A_VEC, GM_TM>(A, a.lda, m0, a.M, kl, a.K, tid, la);
-        gm_load<B_KC, B_VEC, TN>(B, a.ldb, n0, a.N, kl, a.K, tid, lb);
+      for (int u = 0; u < U; ++u) {
+        const uint32_t o = KC ? ((tid >> 2) + 64u * u) * ld4 + k8_of(true, u) * 32u
+                              : (8u * k8_of(false, u) + 2u * q4) * ld4 + (((w + 4u * u) >> 2) * 64u + 4u * c4) * 4u;
+        v[u][0] = gm_bload(r, o);
+        v[u][1] = gm_bload(r, o + (KC ? 16u : ld4));
       }
     } else {
-      gm_load<A_KC, A_VEC, GM_TM, false>(A, a.lda, m0, a.M, kl, a.K, tid, la);
-      gm_load<B_KC, B_VEC, TN, false>(B, a.ldb, n0, a.N, kl, a.K, tid, lb);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int64_t r = r0 + (KC ? (tid >> 2) + 64 * u : ((w + 4 * u) >> 2) * 64 + 4 * c4 + (e & 3));
+          const int64_t k = k0 + 8 * k8_of(KC, u) + (KC ? e : 2 * q4 + (e >> 2));
+          v[u][e >> 2][e & 3] = r < R && k < a.K ? X[KC ? r * ld + k : k * ld + r] : 0.0f;
+        }
     }
-    vh_f4 fa[4][2], fb[4][NTW];
+  };
+  const GmFlag<A_KC> akc{};
+  const GmFlag<B_KC> bkc{};
+  auto load_tile = [&](int64_t k0, int set) {
+    load(akc, GmFlag<A_BUF>{}, A, a.lda, m0, a.M, k0, ra[set]);
+    load(bkc, GmFlag<B_BUF>{}, B, a.ldb, n0, a.N, k0, rb[set]);
+  };
+  // Factors of the pieces: S3_SCALE, negative in every other group of 32 rows of A and
+  // columns of B, and in every other k tile of A: the matrix core's sums drift
+  // towards minus infinity by what they round off (gemm_split.h), which then cancels
+  // along K and over rows and columns.
+  const float fsa = (A_KC ? tid >> 7 : c4 >> 3) & 1 ? -S3_SCALE : S3_SCALE;
+  const float fsb = (B_KC ? tid >> 7 : c4 >> 3) & 1 ? -S3_SCALE : S3_SCALE;
+  auto k_sign = [](int64_t k0) { return k0 & GM_TK ? -1.0f : 1.0f; };
+  // Splits the staged pieces into LDS; k past K (what the loads returned there is
+  // another row's) as zeros, in both operands.
+  auto stage = [&](auto kcv, const vh_f4 (&v)[U][2], uint32_t* S, int64_t k0, float f) {
+    constexpr bool KC = decltype(kcv)::value;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int kc = h * 16 + 4 * q;
-      fa[q][0] = gm_frag<A_KC>(L[sc], wm * 64 + li, kc);
-      fa[q][1] = gm_frag<A_KC>(L[sc], wm * 64 + 32 + li, kc);
+    for (int u = 0; u < U; ++u) {
+      float x[8];
+      if constexpr (KC) {
 #pragma unroll
-      for (int nt = 0; nt < NTW; ++nt) fb[q][nt] = gm_frag<B_KC>(L[2 + sc], wn * (TN / 2) + nt * 32 + li, kc);
-    }
+        for (int e = 0; e < 8; ++e) x[e] = v[u][e >> 2][e & 3];
+      } else {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+        for (int e = 0; e < 2; ++e) {
+          const vh_u4 t4 = __builtin_bit_cast(vh_u4, v[u][e]);
+          uint32_t t[4] = {t4[0], t4[1], t4[2], t4[3]};
+          s3_transpose4(t);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-#pragma unroll
-        for (int nt = 0; nt < NTW; ++nt) {
-          acc[0][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][0][e], fb[q][nt][e], acc[0][nt], 0, 0, 0);
-          acc[1][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][1][e], fb[q][nt][e], acc[1][nt], 0, 0, 0);
+          for (int j = 0; j < 4; ++j) x[2 * j + e] = __builtin_bit_cast(float, t[j]);
         }
       }
-    }
-    gm_store_lds<A_KC, A_VEC, GM_TM>(L[sc ^ 1], tid, wa);
-    gm_store_lds<B_KC, B_VEC, TN>(L[2 + (sc ^ 1)], tid, wb);
-    if constexpr (!CHECK) __builtin_amdgcn_sched_group_barrier(0x020, VM, 0);  // the loads
-    __builtin_amdgcn_sched_group_barrier(0x100, RD, 0);                        // all fragment reads
-    __builtin_amdgcn_sched_group_barrier(0x008, 3 * MF, 0);                    // groups 0-2
+      if (k0 + GM_TK > a.K) {
 #pragma unroll
-    for (int i = 0; i < MF; ++i) {  // group 3 with the writes
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x200, (WR + MF - 1) / MF, 0);
-    }
-    __syncthreads();
-  };
-  // 128 x 128 tiles: the next k tile's loads are in flight during one step
-  // (1.7 us of products). 128 x 64 tiles have half the products per step, less
-  // than the load latency under load, so with 128-bit loads (registers to
-  // spare) theirs run two steps ahead through a second register set: step 0
-  // of a pair computes stage 0, loads k tile k0+64 into (sa, sb) and stages
-  // (sa2, sb2) = k0+32; step 1 the reverse. Unchecked loads past the range
-  // fetch the last k tile again.
-  constexpr bool DEEP = TN == 64 && A_VEC && B_VEC;
-  auto main_loop = [&](auto unchecked) {
-    constexpr bool CHECK = !decltype(unchecked)::value;
-    auto kn = [&](int64_t k) { return CHECK || k < ke ? k : ke - GM_TK; };
-    if constexpr (!DEEP) {
-      for (int64_t k0 = kb; k0 < ke; k0 += GM_TK) {
-        kstep(unchecked, s, sa, sb, sa, sb, kn(k0 + GM_TK), k0 + GM_TK < ke);
-        s ^= 1;
+        for (int e = 0; e < 8; ++e) x[e] = k0 + 8 * k8_of(KC, u) + e < a.K ? x[e] : 0.0f;
       }
-    } else {
-      float sa2[GM_TM / 8] = {}, sb2[TN / 8] = {};
-      if (kb < ke) {
-        if constexpr (CHECK) {
-          if (kb + GM_TK < ke) {
-            gm_load<A_KC, A_VEC, GM_TM>(A, a.lda, m0, a.M, kb + GM_TK, a.K, tid, sa2);
-            gm_load<B_KC, B_VEC, TN>(B, a.ldb, n0, a.N, kb + GM_TK, a.K, tid, sb2);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] *= f;
+      vh_u4 p[3];
+      s3_split8(x, p);
+#pragma unroll
+      for (int t = 0; t < 3; ++t) *reinterpret_cast<vh_u4*>(S + t * 4 * HS + lds_of(KC, u)) = p[t];
+    }
+  };
+  auto lds_barrier = []() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+  vh_f32x16 acc[NW][NW], tt[NW][NW];
+#pragma unroll
+  for (int i = 0; i < NW; ++i)
+#pragma unroll
+    for (int j = 0; j < NW; ++j) acc[i][j] = vh_f32x16{};
+  // Row 32 g + li of an operand's tile: its LDS piece.
+  const int lt = 16 * (li & 3) + (((li >> 2) + 4 * (li & 3)) & 15);
+  auto piece = [&](bool kc, int g) { return kc ? 32 * g + li : 64 * (g >> 1) + (g & 1 ? lt ^ 8 : lt); };
+  vh_u4 fa[2][NW][3], fb[2][NW][3];
+  auto frags = [&](const uint32_t* SA, const uint32_t* SB, int kk) {
+#pragma unroll
+    for (int i = 0; i < NW; ++i)
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        const int o = (4 * t + 2 * kk + h) * HS;
+        fa[kk][i][t] = *reinterpret_cast<const vh_u4*>(SA + o + 4 * piece(A_KC, wm * NW + i));
+        fb[kk][i][t] = *reinterpret_cast<const vh_u4*>(SB + o + 4 * piece(B_KC, wn * NW + i));
+      }
+  };
+  auto products = [&](int kk) {
+#pragma unroll
+    for (int t = 0; t < 6; ++t)
+#pragma unroll
+      for (int i = 0; i < NW; ++i)
+#pragma unroll
+        for (int j = 0; j < NW; ++j)
+          tt[i][j] = s3_mfma(fa[kk][i][S3_PA(t)], fb[kk][j][S3_PB(t)], kk || t ? tt[i][j] : vh_f32x16{});
+  };
+  auto add = [&](float sg) {
+    if (((wm + wn) * NW) & 1) sg = -sg;
+#pragma unroll
+    for (int i = 0; i < NW; ++i)
+#pragma unroll
+      for (int j = 0; j < NW; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(tt[i][j][r], (i ^ j) & 1 ? -sg : sg, acc[i][j][r]);
+  };
+  // Loads past the last k tile fetch it again (every load stays in the range).
+  auto k_at = [&](int st) { return kb + (int64_t)(st < steps ? st : steps - 1) * GM_TK; };
+  if (steps > 0) {
+    if constexpr (D == 2) {
+      // Two stages: k tile st is multiplied from one while st + 1 is split into the
+      // other (free since the barrier: its readers have passed it), its registers
+      // then reloaded with st + 3.
+      load_tile(k_at(0), 0);
+      load_tile(k_at(1), 1);
+      stage(akc, ra[0], L[0][0], k_at(0), fsa * k_sign(kb));
+      stage(bkc, rb[0], L[0][1], k_at(0), fsb);
+      load_tile(k_at(2), 0);
+      for (int st = 0; st < steps; st += 2) {
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+          if (st + d < steps) {
+            lds_barrier();
+            frags(L[d][0], L[d][1], 0);
+            frags(L[d][0], L[d][1], 1);
+            products(0);
+            stage(akc, ra[d ^ 1], L[d ^ 1][0], k_at(st + d + 1), fsa * k_sign(k_at(st + d + 1)));
+            products(1);
+            stage(bkc, rb[d ^ 1], L[d ^ 1][1], k_at(st + d + 1), fsb);
+            load_tile(k_at(st + d + 3), d ^ 1);
+            add(k_sign(k_at(st + d)));
           }
-        } else {
-          gm_load<A_KC, A_VEC, GM_TM, false>(A, a.lda, m0, a.M, kn(kb + GM_TK), a.K, tid, sa2);
-          gm_load<B_KC, B_VEC, TN, false>(B, a.ldb, n0, a.N, kn(kb + GM_TK), a.K, tid, sb2);
         }
       }
-      for (int64_t k0 = kb; k0 < ke; k0 += 2 * GM_TK) {
-        kstep(unchecked, 0, sa, sb, sa2, sb2, kn(k0 + 2 * GM_TK), k0 + 2 * GM_TK < ke);
-        if (k0 + GM_TK >= ke) break;
-        kstep(unchecked, 1, sa2, sb2, sa, sb, kn(k0 + 3 * GM_TK), k0 + 3 * GM_TK < ke);
+    } else {
+      load_tile(k_at(0), 0);
+      for (int st = 0; st < steps; ++st) {
+        stage(akc, ra[0], L[0][0], k_at(st), fsa * k_sign(k_at(st)));
+        stage(bkc, rb[0], L[0][1], k_at(st), fsb);
+        load_tile(k_at(st + 1), 0);
+        lds_barrier();
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          frags(L[0][0], L[0][1], kk);
+          products(kk);
+        }
+        add(k_sign(k_at(st)));
+        lds_barrier();
       }
     }
-  };
-  const bool inside = m0 + GM_TM <= a.M && n0 + TN <= a.N && (ke - kb) % GM_TK == 0 && ke <= a.K;
-  if (inside)
-    main_loop(GmFlag<true>{});
-  else
-    main_loop(GmFlag<false>{});
+  }
+#pragma unroll
+  for (int i = 0; i < NW; ++i)
+#pragma unroll
+    for (int j = 0; j < NW; ++j) acc[i][j] *= S3_UNSCALE;
+  if (tiny || s3_nonfinite(acc)) {
+    // On the f32 instruction, straight from memory (see split3.h).
+#pragma unroll
+    for (int i = 0; i < NW; ++i)
+#pragma unroll
+      for (int j = 0; j < NW; ++j) acc[i][j] = vh_f32x16{};
+#pragma nounroll
+    for (int64_t k0 = kb; k0 < ke; k0 += 2) {
+      const int64_t k = k0 + h;
+      float xa[NW], xb[NW];
+#pragma unroll
+      for (int i = 0; i < NW; ++i) {
+        const int64_t m = m0 + wm * (T / 2) + 32 * i + li, n = n0 + wn * (T / 2) + 32 * i + li;
+        xa[i] = m < a.M && k < ke ? A[A_KC ? m * a.lda + k : k * a.lda + m] : 0.0f;
+        xb[i] = n < a.N && k < ke ? B[B_KC ? n * a.ldb + k : k * a.ldb + n] : 0.0f;
+      }
+#pragma unroll
+      for (int i = 0; i < NW; ++i)
+#pragma unroll
+        for (int j = 0; j < NW; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[i], xb[j], acc[i][j], 0, 0, 0);
+    }
+  }
 
-  // Epilogue. Straight from the accumulators, one wave store covers two
-  // 128-byte row pieces; a tile wholly inside C with 16-byte aligned rows goes
-  // through LDS instead (the k loop's last barrier has freed it), so that each
-  // store writes 16 bytes and a half-wave a whole 512-byte row.
-  float* out = split ? a.ws + (int64_t)blockIdx.y * a.M * a.N : C;
-  const int64_t ldo = split ? a.N : a.ldc;
+  float* out = split ? a.ws + (int64_t)kr * a.M * a.N : C;
   const float* E0 = gm_addend(a);
   const float* E = !split && E0 ? E0 + b1 * a.se1 + b2 * a.se2 : nullptr;
-  const bool whole = m0 + GM_TM <= a.M && n0 + TN <= a.N && (ldo & 3) == 0 &&
-                     (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-  if (whole) {
-    constexpr int CS = TN + 8;  // row stride (floats): rows 4 apart are 32 banks apart
-    static_assert(GM_TM * CS <= 4 * GM_STAGE, "C tile fits the operand LDS");
-    float* Cs = &L[0][0];
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < NTW; ++nt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          Cs[(wm * 64 + mt * 32 + 8 * (r >> 2) + 4 * h + (r & 3)) * CS + wn * (TN / 2) + nt * 32 + li] =
-              acc[mt][nt][r];
-    __syncthreads();
-    constexpr int Q = TN / 4;      // 16-byte pieces per row
-    constexpr int RP = 256 / Q;    // rows per pass
-    const int c = (tid % Q) * 4, r0 = tid / Q;
-#pragma unroll 4
-    for (int i = 0; i < GM_TM / RP; ++i) {
-      const int row = r0 + RP * i;
-      const int64_t m = m0 + row, n = n0 + c;
-      vh_f4 v = *reinterpret_cast<const vh_f4*>(Cs + row * CS + c);
-      vh_f4* op = reinterpret_cast<vh_f4*>(out + m * ldo + n);
-      if (!split) {
-        const vh_f4 old = a.accumulate ? *op : vh_f4{};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = gm_finish(a, E, false, v[e], m, n + e, old[e]);
-      }
-      *op = v;
-    }
-    return;
-  }
-  gm_store_direct<NTW>(a, acc, out, ldo, E, split, m0, n0, wm, wn, li, h);
+  gm_store_direct<NW, NW>(a, acc, out, split ? a.N : a.ldc, E, split, m0, n0, T, wm, wn, li, h);
 }
 
 // Persistent form for batched products with a short k range (attention's
@@ -558,7 +677,7 @@ VH_DEV void gemm_f32_persist(const GemmArgs& a) {
       k_loop(GmFlag<false>{});
     // Streaming stores: with normal ones the write of a score-sized output
     // runs at ~1.8 TB/s here, with these at ~2.8 TB/s (measured).
-    gm_store_direct<NTW, true>(a, acc, cur.C, a.ldc, cur.E, false, cur.m0, cur.n0, wm, wn, li, h);
+    gm_store_direct<2, NTW, true>(a, acc, cur.C, a.ldc, cur.E, false, cur.m0, cur.n0, GM_TM, wm, wn, li, h);
     if (!has_next) break;
     item = nit;
     cur = nxt;

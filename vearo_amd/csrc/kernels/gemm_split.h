@@ -58,20 +58,6 @@
 #define GS_PART (2 * GS_HALF)    // dwords per part
 #define GS_STAGE (3 * GS_PART)   // dwords per operand and stage
 
-// Buffer resource from `org` covering `bytes` bytes, clamped to [0, 2^32 - 1]
-// from the two 32-bit halves (gb_rsrc's clamp; here the halves are hidden from
-// the compiler, which otherwise joins them again into a 64-bit vector compare
-// once per k step).
-VH_DEV __amdgpu_buffer_rsrc_t gs_rsrc(const float* org, int64_t bytes) {
-  uint32_t hi = (uint32_t)((uint64_t)bytes >> 32), lo = (uint32_t)bytes;
-  asm("" : "+s"(hi), "+s"(lo));  // keeps the compiler from joining the halves again
-  const uint32_t nrec = (int32_t)hi < 0 ? 0u : (hi != 0 ? 0xFFFFFFFFu : lo);
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(org), (short)0, (int)nrec, GB_RSRC_W3);
-}
-VH_DEV vh_f4 gs_load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  return __builtin_bit_cast(vh_f4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-}
-
 // The work split shared by the kernel and the fix-up: G workgroups, `full`
 // whole-tile rounds, then W = rem * nk k tiles split evenly (the host keeps
 // tile and k tile counts, and W, below 2^31). With a.whole_tail the rem tiles
@@ -264,10 +250,10 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
   // (The offsets are opaque at each use: the second load's is then formed there,
   // as the instruction's immediate or one addition, instead of held in a register.)
   auto load2 = [](const char* p, int64_t n, uint32_t o, uint32_t o2, vh_f4 (&v)[2]) {
-    const auto r = gs_rsrc(reinterpret_cast<const float*>(p), n);
+    const auto r = gm_rsrc(reinterpret_cast<const float*>(p), n);
     asm volatile("" : "+v"(o));
-    v[0] = gs_load(r, o);
-    v[1] = gs_load(r, o + o2);
+    v[0] = gm_bload(r, o);
+    v[1] = gm_bload(r, o + o2);
   };
   auto load_a = [&]() { load2(pa, na, oa, oa2, ga); };
   auto load_b = [&]() { load2(pb, nb, ob, ob2, gb); };

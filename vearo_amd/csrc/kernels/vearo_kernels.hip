@@ -218,14 +218,15 @@ extern "C" __global__ void __launch_bounds__(256) vh_fill(FillArgs a) { fill_imp
 extern "C" __global__ void __launch_bounds__(256) vh_math_probe(MathProbeArgs a) { math_probe_impl(a); }
 extern "C" __global__ void __launch_bounds__(256) vh_stream_copy(StreamCopyArgs a) { stream_copy_impl(a); }
 
-// Matrix multiply: vh_gemm_<A><B>, each operand k-contiguous ("k") or
-// m/n-contiguous ("m"/"n"), with 128-bit ("4") or 32-bit ("1") global loads.
+// Matrix multiply: vh_gemm_<A><B>[_t64], 128 x 128 or 64 x 64 tiles, each operand
+// k-contiguous ("k") or m/n-contiguous ("m"/"n"), through 128-bit buffer loads ("4")
+// or, where their 32-bit offsets do not reach, element by element ("1").
 #define K_GEMM(AK, AV, BK, BV, NAME)                                                            \
   extern "C" __global__ void __launch_bounds__(256, 2) NAME(GemmArgs a) {                      \
-    gemm_f32_impl<AK, AV, BK, BV, 128>(a);                                                      \
+    gemm_tile_impl<AK, AV, BK, BV, 128>(a);                                                     \
   }                                                                                             \
   extern "C" __global__ void __launch_bounds__(256, 2) NAME##_t64(GemmArgs a) {                \
-    gemm_f32_impl<AK, AV, BK, BV, 64>(a);                                                       \
+    gemm_tile_impl<AK, AV, BK, BV, 64>(a);                                                      \
   }
 K_GEMM(true, true, true, true, vh_gemm_k4_k4)
 K_GEMM(true, true, true, false, vh_gemm_k4_k1)
@@ -243,6 +244,14 @@ K_GEMM(false, false, true, true, vh_gemm_m1_k4)
 K_GEMM(false, false, true, false, vh_gemm_m1_k1)
 K_GEMM(false, false, false, true, vh_gemm_m1_n4)
 K_GEMM(false, false, false, false, vh_gemm_m1_n1)
+// The 64 x 64 tiles walked by resident workgroups (products short of filling the
+// 256-row kernels).
+#define K_GEMMT(AK, BK, NAME) \
+  extern "C" __global__ void __launch_bounds__(256, 2) NAME(GemmArgs a) { gemm_tile_walk<AK, BK, 64>(a); }
+K_GEMMT(true, true, vh_gemmt_kk)
+K_GEMMT(true, false, vh_gemmt_kn)
+K_GEMMT(false, true, vh_gemmt_mk)
+K_GEMMT(false, false, vh_gemmt_mn)
 // Persistent form of the 128-bit-load layouts (batched products with short k).
 #define K_GEMMP(AK, BK, NAME) \
   extern "C" __global__ void __launch_bounds__(256, 2) NAME(GemmArgs a) { gemm_f32_persist<AK, true, BK, true>(a); }

@@ -1372,46 +1372,46 @@ static bool gemm_vec_ok(const float* p, int64_t ld, int64_t ext, const int64_t* 
   return aligned16(p) && ld % 4 == 0 && ext % 4 == 0 && sb[0] % 4 == 0 && sb[1] % 4 == 0;
 }
 
+// Operands the tiled kernel reads through buffer loads: 4-byte-aligned bases, and a
+// tile's byte offsets (128 rows, or 32 k rows of `ld`) within 32 bits.
+static bool gemm_buf_ok(const float* p, int64_t ld) {
+  return reinterpret_cast<uintptr_t>(p) % 4 == 0 && ld < (int64_t(1) << 22);
+}
+
 namespace {
 struct GemmPlan {
-  bool narrow;     // 128 x 64 C tiles instead of 128 x 128
+  int64_t tile;    // 128 x 128 or 64 x 64 C tiles
   int64_t ksplit;  // K ranges, each its own workgroups; 1 = no split
   int64_t kchunk;  // k per range, a multiple of the 32-wide k tile
+  double us;       // the estimate the choice was made by
 };
 
-// Tile width and split-K for a product: the shape whose estimated time is
-// least. A split or a narrow tile pays where the C tiles leave the chip's
-// resident workgroups (2 per CU) idle -- a last wave mostly empty (768 tiles on
-// 512 slots) or too few tiles to fill it (the weight gradients, 768 x 768
-// outputs over K = 16384 rows). Time is counted in k steps of one 128-wide
-// tile: waves x tile width x (k per range + a fixed cost for the prologue and
-// epilogue), a narrow tile at 0.88 of the wide one's matrix-core rate (its B
-// fragments feed half as many products), plus the fixed-order reduce of the
-// split partials ((ks + 1) M N floats through HBM). Batched and causal
-// products do not split. N <= 64 (attention's P v and its gradients,
-// N = Dk = 64) always takes the narrow tile.
-GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
-  const int64_t slots = 2 * std::max(g_rt.cu_count, 1);
-  GemmPlan best{N <= VH_GEMM_TILE_N / 2, 1, K};
-  if (!may_split || K == 0) return best;
-  double best_t = -1.0;
-  for (int tn : {VH_GEMM_TILE_N, VH_GEMM_TILE_N / 2}) {
-    if (N <= VH_GEMM_TILE_N / 2 && tn != VH_GEMM_TILE_N / 2) continue;
-    const int64_t tiles = cdiv(M, VH_GEMM_TILE_M) * cdiv(N, tn);
+// Tile and split of K for a product on the tiled kernel (`nb` batches; they and
+// causal products do not split): the shape whose estimated time is least. Measured
+// on MI355X, a k tile (32) of a 64 x 64 workgroup takes 0.8 us with one workgroup on
+// its CU, 1.15 with two, 1.55 with three (its LDS allows no more), and 0.53 us a
+// workgroup past that; of a 128 x 128 one 2.25 us, 3.3 with two, 1.65 past that; a
+// launch 2.5 us; a split adds the reduce, 4 us and (ks + 1) M N floats at 4 TB/s.
+// [1000, 768] x [768, 768], 64-wide, ks = 1 / 2 / 4: 22.3 / 21.8 / 22.3 us; 128-wide 58 /
+// 38 / 30; [256, 128] x [128, 384] 5.8 (128-wide 10.9); [4096, 768] x [768, 768] 40.8 (53);
+// [2048, 500] x [500, 3000] 58 (56); [600, 3000] x [3000, 600], ks = 1 / 2 / 4 / 6 / 8: 80 / 46 /
+// 34 / 33 / 37. Attention's P v (192 x [1024, 1024] x [1024, 64]) 249 us (128-wide 364).
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int64_t nb, bool may_split) {
+  const double cus = std::max(g_rt.cu_count, 1);
+  GemmPlan best{0, 1, K, 0.0};
+  for (int64_t tile : {int64_t(64), int64_t(VH_GEMM_TILE_M)}) {
+    const double tiles = (double)cdiv(M, tile) * (double)cdiv(N, tile) * (double)nb;
     for (int64_t want = 1; want <= 32; ++want) {
-      if (want > 1 && K / want < 256) break;
-      const int64_t kchunk = cdiv(cdiv(K, want), 32) * 32;
-      const int64_t ks = cdiv(K, kchunk);
+      if (want > 1 && (!may_split || K / want < 64)) break;
+      const int64_t kchunk = std::max<int64_t>(32, cdiv(cdiv(K, want), 32) * 32);
+      const int64_t ks = std::max<int64_t>(1, cdiv(K, kchunk));
       if (ks != want) continue;
-      const int64_t n = tiles * ks;
-      const double waves = (double)cdiv(n, slots);  // a part-filled last wave costs a whole one
-      double t = waves * ((double)tn / VH_GEMM_TILE_N) * ((double)kchunk + 48.0) /
-                 (tn == VH_GEMM_TILE_N ? 1.0 : 0.88);
-      if (ks > 1) t += (double)(ks + 1) * (double)M * (double)N * 4.0 / 536e3;
-      if (best_t < 0.0 || t < best_t) {
-        best_t = t;
-        best = GemmPlan{tn != VH_GEMM_TILE_N, ks, kchunk};
-      }
+      const double n = tiles * (double)ks / cus;  // workgroups per CU
+      const double step = tile == 64 ? (n <= 1 ? 0.8 : n <= 2 ? 1.15 : n <= 3 ? 1.55 : 0.53 * n)
+                                     : (n <= 1 ? 2.25 : n <= 2 ? 3.3 : 1.65 * n);
+      double us = 2.5 + (double)(kchunk / 32) * step;
+      if (ks > 1) us += 4.0 + (double)(ks + 1) * (double)M * (double)N * 1e-6;
+      if (!best.tile || us < best.us) best = GemmPlan{tile, ks, ks > 1 ? kchunk : K, us};
     }
   }
   return best;
@@ -1507,6 +1507,41 @@ bool gemm_persistent_ok(const vh_gemm_desc* d, int64_t lda, int64_t ldb) {
          (double)cdiv(M, VH_GEMMB_TM) * (double)cdiv(N, VH_GEMMB_TN) * (double)nb < (double)INT32_MAX;
 }
 
+// A product split along K on the tiled kernel `name` (grid gx x gy): raw partials, then
+// the fixed-order reduce, which applies alpha, the addend and accumulation.
+int gemm_split_k(const vh_gemm_desc* d, const GemmPlan& plan, int64_t lda, int64_t ldb, const std::string& name,
+                 int64_t gx, int64_t gy, hipStream_t s) {
+  const int64_t M = d->M, N = d->N, ks = plan.ksplit;
+  void* ws = nullptr;
+  VH_TRY(g_arena.alloc((size_t)(ks * M * N) * sizeof(float), s, &ws));
+  GemmArgs g = gemm_args(d, lda, ldb, cdiv(M, plan.tile), cdiv(N, plan.tile));
+  g.E = nullptr;
+  g.accumulate = 0;
+  g.nbat = 1;
+  g.ksplit = (int32_t)ks;
+  g.kchunk = plan.kchunk;
+  g.ws = static_cast<float*>(ws);
+  int rc = launch(name, gx, gy, 256, 0, s, g);
+  if (rc == VH_OK) {
+    GemmReduceArgs r{g.ws, d->c, d->e, M, N, d->c_sm, d->e_sm, d->e_sn, (int32_t)ks, d->accumulate ? 1 : 0, d->alpha};
+    rc = launch("vh_gemm_reduce", std::min<int64_t>(cdiv(M * N, 256), 8192), 1, 256, 0, s, r);
+  }
+  g_arena.free(ws, s);
+  return rc;
+}
+
+// The 64 x 64 tiles walked by resident workgroups (three per CU).
+int gemm_walk(const vh_gemm_desc* d, const GemmPlan& plan, bool akc, bool bkc, int64_t lda, int64_t ldb,
+              hipStream_t s) {
+  const int64_t nb = d->batch[0] * d->batch[1], tiles_m = cdiv(d->M, plan.tile), tiles_n = cdiv(d->N, plan.tile);
+  const int64_t grid = std::min<int64_t>(tiles_m * tiles_n * plan.ksplit * nb, 3 * std::max(g_rt.cu_count, 1));
+  const std::string name = std::string("vh_gemmt_") + (akc ? "k" : "m") + (bkc ? "k" : "n");
+  if (plan.ksplit > 1) return gemm_split_k(d, plan, lda, ldb, name, grid, 1, s);
+  GemmArgs g = gemm_args(d, lda, ldb, tiles_m, tiles_n);
+  g.nbat = nb;
+  return launch(name, grid, 1, 256, 0, s, g);
+}
+
 // One launch of the split persistent kernel (and its fix-up).
 int gemm_split_range(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t ldb, hipStream_t s) {
   const int64_t M = d->M, N = d->N, K = d->K, nb = d->batch[0] * d->batch[1];
@@ -1545,6 +1580,20 @@ int gemm_split_range(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int
 int gemm_split(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t ldb, hipStream_t s, bool* taken) {
   *taken = false;
   if (!gemm_persistent_ok(d, lda, ldb)) return VH_OK;
+  // Below ~1e9 multiply-adds the 256-row tiles are too few or their pieces too many:
+  // the 64 x 64 tiles where their estimate is less ([1000, 768] x [768, 768]: 36.7 us
+  // with its fix-up against 22.3; 5 us of launches are added to the other's).
+  const int64_t nb = d->batch[0] * d->batch[1];
+  if (d->K <= 16384 && (double)cdiv(d->M, 64) * (double)cdiv(d->N, 64) * (double)nb < 1e6) {
+    const GemmPlan tiled = gemm_plan(d->M, d->N, d->K, nb, nb == 1);
+    const int G = std::max(8, g_rt.cu_count / 8 * 8);
+    if (tiled.tile == 64 && tiled.us < gemm_split_plan(d->M, d->N, d->K, nb, G).us + 5.0) {
+      VH_TRY(gemm_walk(d, tiled, akc, bkc, lda, ldb, s));
+      *taken = true;
+      g_gemm_path = VH_GEMM_PATH_PERSISTENT;
+      return VH_OK;
+    }
+  }
   const int64_t K = d->K, n = K > 16384 ? cdiv(K, 8192) : 1;
   const int64_t kc = cdiv(cdiv(K, n), VH_GEMMS_TK) * VH_GEMMS_TK;
   for (int64_t k0 = 0; k0 < K; k0 += kc) {
@@ -1668,55 +1717,38 @@ int vh_gemm(const vh_gemm_desc* d, void* stream) {
     VH_TRY((d->engine == VH_GEMM_ENGINE_WIDE ? gemm_big : gemm_split)(d, akc, bkc, lda, ldb, S(stream), &taken));
     if (taken) return VH_OK;
   }
-  const bool avec = K > 0 && gemm_vec_ok(d->a, lda, akc ? K : M, d->a_sb);
-  const bool bvec = K > 0 && gemm_vec_ok(d->b, ldb, bkc ? K : N, d->b_sb);
-  const GemmPlan plan = gemm_plan(M, N, K, !dflag && d->batch[0] * d->batch[1] == 1 && d->causal == VH_GEMM_DENSE);
-  const int64_t tiles_m = cdiv(M, VH_GEMM_TILE_M), tiles_n = cdiv(N, plan.narrow ? 64 : VH_GEMM_TILE_N);
+  const int64_t nbat = d->batch[0] * d->batch[1];
+  const GemmPlan plan =
+      gemm_plan(M, N, K, nbat, K > 0 && !dflag && nbat == 1 && d->causal == VH_GEMM_DENSE);
+  const int64_t tiles_m = cdiv(M, plan.tile), tiles_n = cdiv(N, plan.tile);
   if (tiles_m * tiles_n > INT32_MAX) return fail(VH_ERR_UNSUPPORTED, "vh_gemm: too many tiles");
-  const std::string name = std::string("vh_gemm_") + (akc ? "k" : "m") + (avec ? "4" : "1") + "_" +
-                           (bkc ? "k" : "n") + (bvec ? "4" : "1") + (plan.narrow ? "_t64" : "");
+  const std::string name = std::string("vh_gemm_") + (akc ? "k" : "m") + (gemm_buf_ok(d->a, lda) ? "4" : "1") + "_" +
+                           (bkc ? "k" : "n") + (gemm_buf_ok(d->b, ldb) ? "4" : "1") + (plan.tile == 64 ? "_t64" : "");
   hipStream_t s = S(stream);
-  const int64_t tiles = tiles_m * tiles_n;
-  {
-    const int64_t ks = plan.ksplit, kchunk = plan.kchunk;
-    if (ks > 1) {
-      void* ws = nullptr;
-      VH_TRY(g_arena.alloc((size_t)(ks * M * N) * sizeof(float), s, &ws));
-      // Raw partials: the reduce applies alpha, the addend and accumulation.
-      GemmArgs g = gemm_args(d, lda, ldb, tiles_m, tiles_n);
-      g.E = nullptr;
-      g.accumulate = 0;
-      g.ksplit = (int32_t)ks;
-      g.kchunk = kchunk;
-      g.ws = static_cast<float*>(ws);
-      int rc = launch(name, tiles, ks, 256, 0, s, g);
-      if (rc == VH_OK) {
-        GemmReduceArgs r{g.ws, d->c, d->e, M, N, d->c_sm, d->e_sm, d->e_sn, (int32_t)ks,
-                         d->accumulate ? 1 : 0, d->alpha};
-        const int64_t blocks = std::min<int64_t>(cdiv(M * N, 256), 8192);
-        rc = launch("vh_gemm_reduce", blocks, 1, 256, 0, s, r);
-      }
-      g_arena.free(ws, s);
-      if (rc == VH_OK) g_gemm_path = VH_GEMM_PATH_SPLIT_K;
-      return rc;
-    }
+  if (plan.ksplit > 1) {
+    VH_TRY(gemm_split_k(d, plan, lda, ldb, name, tiles_m * tiles_n, plan.ksplit, s));
+    g_gemm_path = VH_GEMM_PATH_SPLIT_K;
+    return VH_OK;
   }
   // Batched products with a short k range (attention's q k^T and dO v^T,
   // K = Dk): one workgroup per resident slot walks the tiles of all batches,
   // loading each tile's operands under the previous tile's products
   // (gemm_f32_persist). A workgroup per tile spends most of its short life
   // waiting for its first loads there.
-  const int64_t nbat = d->batch[0] * d->batch[1];
-  if (nbat > 1 && K > 0 && K <= 256 && avec && bvec && !plan.narrow &&
-      (d->causal == VH_GEMM_DENSE || (d->causal == VH_GEMM_SKIP_UPPER && tiles_n >= tiles_m))) {
-    GemmArgs g = gemm_args(d, lda, ldb, tiles_m, tiles_n);
+  // It pays from more than one round of its 128 x 128 tiles on the resident
+  // slots (24 x [333, 64] x [64, 333]: 25 us against 13 for 64 x 64 tiles; 192 causal
+  // [1024, 64] x [64, 1024]: 173 against 238).
+  const int64_t pm = cdiv(M, VH_GEMM_TILE_M), pn = cdiv(N, VH_GEMM_TILE_N);
+  const int64_t slots = 8 * std::max<int64_t>(1, 2 * std::max(g_rt.cu_count, 1) / 8);
+  // (Counted dense whatever the mode: the dense, causal and device-decided forms of
+  // an attention call take the same kernel, and so give the same bits.)
+  if (nbat > 1 && K > 0 && K <= 256 && N > VH_GEMM_TILE_N / 2 && pm * pn * nbat > slots &&
+      gemm_vec_ok(d->a, lda, akc ? K : M, d->a_sb) && gemm_vec_ok(d->b, ldb, bkc ? K : N, d->b_sb) &&
+      (d->causal == VH_GEMM_DENSE || (d->causal == VH_GEMM_SKIP_UPPER && pn >= pm))) {
+    GemmArgs g = gemm_args(d, lda, ldb, pm, pn);
     g.nbat = nbat;
-    // Under a device flag the product may run dense: size the grid for that.
-    const int64_t live = (d->causal == VH_GEMM_SKIP_UPPER && !dflag) ? tiles_m * (tiles_m + 1) / 2 : tiles;
-    const int64_t slots = 8 * std::max<int64_t>(1, 2 * std::max(g_rt.cu_count, 1) / 8);
-    const int64_t grid = std::min<int64_t>(slots, 8 * cdiv(live * nbat, 8));
     const std::string pname = std::string("vh_gemmp_") + (akc ? "k4" : "m4") + "_" + (bkc ? "k4" : "n4");
-    VH_TRY(launch(pname, grid, 1, 256, 0, s, g));
+    VH_TRY(launch(pname, slots, 1, 256, 0, s, g));
     g_gemm_path = VH_GEMM_PATH_BATCHED;
     return VH_OK;
   }
