@@ -203,3 +203,36 @@ def test_tiled_product_far_apart_rows(vh, akc):
     ref = a.astype(np.float64) @ b.astype(np.float64)
     bound = (K + 2) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))
     assert np.all(np.abs(fetch(vh, C, (M, N)) - ref) <= bound)
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+@pytest.mark.parametrize("akc,bkc", LAYOUTS)
+@pytest.mark.parametrize("K", [4, 8, 12, 32, 36, 64, 256])
+def test_streamed_tiles(vh, akc, bkc, K, causal):
+    """Batched short-K products as a stream of 128 x 128 tiles: edge tiles, one to
+    eight k tiles and a ragged last one, K <= 8 on the f32 instruction, an infinity
+    and a NaN in one batch (their own outputs alone), more tiles than workgroups."""
+    nb, M, N = 140, 132, 260
+    print("stream", akc, bkc, K, causal, flush=True)
+    r = np.random.default_rng(K)
+    a = r.standard_normal((nb, M, K)).astype(np.float32)
+    b = r.standard_normal((nb, K, N)).astype(np.float32)
+    a[77, 130, 2], a[77, 3, 1] = np.inf, np.nan
+    A = dev(vh, np.ascontiguousarray(a if akc else np.swapaxes(a, 1, 2)))
+    B = dev(vh, np.ascontiguousarray(np.swapaxes(b, 1, 2) if bkc else b))
+    C = out(vh, (nb, M, N))
+    d = gemm_desc(vh, M, N, K, A.ptr, K if akc else 1, 1 if akc else M, B.ptr, 1 if bkc else N, K if bkc else 1,
+                  C.ptr, N, batch=(nb // 10, 10), a_sb=(10 * M * K, M * K), b_sb=(10 * K * N, K * N),
+                  c_sb=(10 * M * N, M * N), causal=vh.GEMM_SKIP_UPPER if causal else 0)
+    vh.check(vh.lib.vh_gemm(ctypes.byref(d), None))
+    assert vh.lib.vh_gemm_last_path() == vh.GEMM_PATH_BATCHED
+    got = fetch(vh, C, (nb, M, N))
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        ref, mag = a64 @ b64, np.abs(a64) @ np.abs(b64)
+    u = 2.0 ** -24
+    keep = np.tril(np.ones((M, N), bool)) if causal else np.ones((M, N), bool)  # (what causal = 1 defines)
+    fine = np.isfinite(ref) & keep
+    assert np.all(np.abs(got - ref)[fine] <= (K * u / (1 - K * u)) * mag[fine])
+    odd = ~np.isfinite(ref) & keep
+    np.testing.assert_array_equal(got[odd], ref[odd].astype(np.float32))

@@ -1,4 +1,5 @@
-// gemm.h -- f32 matrix multiply on the gfx950 matrix cores (v_mfma_f32_32x32x2_f32).
+// gemm.h -- f32 matrix multiply on the gfx950 matrix cores, each operand value split
+// in three bf16 parts (split3.h).
 //
 // Semantics: vearo-backend-cpu matmul (crates/vearo-backend-cpu/src/lib.rs:266-417),
 // C[m, n] = sum_k A[m, k] * B[k, n] in f32 (the matrix core accumulates in f32;
@@ -9,20 +10,9 @@
 // `* scale` and `+ mask` in attention (cpu:2431-2449), `+ bias` in Linear
 // (nn:120-128), and gradient accumulation `existing.add(g)` (autograd:733-742).
 //
-// Tiling: a 256-thread workgroup computes a 128 x TN tile of C (TN = 128, or
-// 64 for the attention products with N = Dk = 64); its 4 waves own 64 x TN/2
-// quadrants as 2 x TN/64 matrix-core tiles of 32 x 32. K advances in
-// tiles of 32, double-buffered through LDS: the global loads of tile t+1 are in
-// flight while tile t is multiplied. LDS keeps each operand in the orientation
-// of its HBM layout, so staging is 128-bit and bank-conflict free both ways:
-// a k-contiguous operand as [row][k] (rows padded to 36 floats), read as 128-bit
-// fragments; a row-contiguous one (a transposed view) as [k][row] (132 floats
-// per k), read 32 bits at a time with consecutive lanes on consecutive rows.
-// Lane half h (lanes 32h..32h+31) takes k in [16h, 16h+16) of the tile, step s
-// pairing k = s with k = 16 + s.
+// Tiling: GemmTile below, 128 x 128 or 64 x 64 C tiles; K in tiles of 32.
 // A operand layouts: k-contiguous (A[m, k] at m*lda + k) or m-contiguous
-// (A[m, k] at k*lda + m, a transposed view); the same for B. Global loads are
-// 128-bit when the layout allows (host-checked alignment), else 32-bit.
+// (A[m, k] at k*lda + m, a transposed view); the same for B.
 //
 // Causal modes for attention's score blocks (the masked part is exactly 0 or
 // never read, so skipping it changes no result):
@@ -35,97 +25,12 @@
 
 #define GM_TM VH_GEMM_TILE_M
 #define GM_TK 32
-#define GM_LS (GM_TK + 4)  // [row][k] LDS row stride (floats): 16-byte aligned rows, staggered banks
-#define GM_LT (GM_TM + 4)  // [k][row] LDS stride (floats)
-#define GM_STAGE (GM_TM * GM_LS > GM_TK * GM_LT ? GM_TM * GM_LS : GM_TK * GM_LT)  // one 128-row operand tile
 #define GM_GROUP 8         // tile rows per group in the launch order (L2 reuse of B)
 
 template <bool B>
 struct GmFlag {
   static constexpr bool value = B;
 };
-
-// The [NR rows x 32 k] tile (NR = 128 or 64) whose element (r, k) is at
-//   KC:  base[(r0 + r) * ld + k0 + k]      !KC: base[(k0 + k) * ld + r0 + r]
-// into NR/8 staging registers per thread; rows >= R or k >= K read as 0.
-// VEC requires 16-byte aligned base and ld, and K (KC) or R (!KC) % 4 == 0.
-// CHECK = false: the caller knows the whole tile is inside (no tests, no
-// branches: the loads can be scheduled among the matrix-core products).
-template <bool KC, bool VEC, int NR, bool CHECK = true>
-VH_DEV void gm_load(const float* base, int64_t ld, int64_t r0, int64_t R, int64_t k0, int64_t K, int tid,
-                    float (&st)[NR / 8]) {
-  if constexpr (KC && VEC) {
-#pragma unroll
-    for (int i = 0; i < NR / 32; ++i) {
-      const int r = (tid >> 3) + 32 * i, k = (tid & 7) * 4;
-      vh_f4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (!CHECK || (r0 + r < R && k0 + k < K)) v = *reinterpret_cast<const vh_f4*>(base + (r0 + r) * ld + k0 + k);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) st[4 * i + e] = v[e];
-    }
-  } else if constexpr (KC) {
-#pragma unroll
-    for (int i = 0; i < NR / 8; ++i) {
-      const int r = (tid >> 5) + 8 * i, k = tid & 31;
-      st[i] = (!CHECK || (r0 + r < R && k0 + k < K)) ? base[(r0 + r) * ld + k0 + k] : 0.0f;
-    }
-  } else if constexpr (VEC) {
-    constexpr int TPR = NR / 4;  // threads per k row
-#pragma unroll
-    for (int i = 0; i < NR / 32; ++i) {
-      const int k = tid / TPR + (256 / TPR) * i, r = (tid % TPR) * 4;
-      vh_f4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (!CHECK || (k0 + k < K && r0 + r < R)) v = *reinterpret_cast<const vh_f4*>(base + (k0 + k) * ld + r0 + r);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) st[4 * i + e] = v[e];
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < NR / 8; ++i) {
-      const int k = tid / NR + (256 / NR) * i, r = tid % NR;
-      st[i] = (!CHECK || (k0 + k < K && r0 + r < R)) ? base[(k0 + k) * ld + r0 + r] : 0.0f;
-    }
-  }
-}
-
-template <bool KC, bool VEC, int NR>
-VH_DEV void gm_store_lds(float* S, int tid, const float (&st)[NR / 8]) {
-  if constexpr (KC && VEC) {
-#pragma unroll
-    for (int i = 0; i < NR / 32; ++i) {
-      const int r = (tid >> 3) + 32 * i, k = (tid & 7) * 4;
-      vh_f4 v = {st[4 * i], st[4 * i + 1], st[4 * i + 2], st[4 * i + 3]};
-      *reinterpret_cast<vh_f4*>(S + r * GM_LS + k) = v;
-    }
-  } else if constexpr (KC) {
-#pragma unroll
-    for (int i = 0; i < NR / 8; ++i) S[((tid >> 5) + 8 * i) * GM_LS + (tid & 31)] = st[i];
-  } else if constexpr (VEC) {
-    constexpr int TPR = NR / 4;
-#pragma unroll
-    for (int i = 0; i < NR / 32; ++i) {
-      const int k = tid / TPR + (256 / TPR) * i, r = (tid % TPR) * 4;
-      vh_f4 v = {st[4 * i], st[4 * i + 1], st[4 * i + 2], st[4 * i + 3]};
-      *reinterpret_cast<vh_f4*>(S + k * GM_LT + r) = v;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < NR / 8; ++i) S[(tid / NR + (256 / NR) * i) * GM_LT + tid % NR] = st[i];
-  }
-}
-
-// Fragment of row `row` for k = k0 .. k0+3 (4 matrix-core steps).
-template <bool KC>
-VH_DEV vh_f4 gm_frag(const float* S, int row, int k0) {
-  if constexpr (KC) {
-    return *reinterpret_cast<const vh_f4*>(S + row * GM_LS + k0);
-  } else {
-    vh_f4 f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) f[e] = S[(k0 + e) * GM_LT + row];
-    return f;
-  }
-}
 
 // Workgroup -> C tile. Workgroups are dealt to the 8 XCDs round-robin; this
 // gives each XCD a contiguous run of tile ids, and runs of GM_GROUP tile rows
@@ -259,8 +164,33 @@ struct GemmTile {
   static constexpr int HS = T * 4 + 16, OP = 12 * HS;  // dwords per k eighth (64 bytes of padding), per operand
   static constexpr int D = T == 64 ? 2 : 1;            // LDS stages
   using Lds = uint32_t[D][2][OP];
+  // The staging registers (a k tile of each operand), and where a tile's first k tile is.
+  struct Regs {
+    vh_f4 a[D][T / 64][2], b[D][T / 64][2];
+  };
+  struct Origin {
+    const float *A, *B;
+    int64_t m0, n0;
+  };
   // C tile (tm, tn) of batch `bat`, or its raw partial over K range `kr` of a.ksplit.
-  static VH_DEV void run(const GemmArgs& a, Lds& L, int tm, int tn, int64_t bat, int kr, int causal);
+  // STREAM (T = 128, no split): R holds the tile's first k tile already, and the last k
+  // step loads the one at `next` (null: none) into it; streaming stores.
+  template <bool STREAM = false>
+  static VH_DEV void run(const GemmArgs& a, Lds& L, int tm, int tn, int64_t bat, int kr, int causal, Regs& R,
+                         const Origin* next = nullptr);
+  static VH_DEV Origin origin(const GemmArgs& a, int tm, int tn, int64_t bat) {
+    const int64_t b1 = bat / a.nb2, b2 = bat % a.nb2;
+    return Origin{a.A + b1 * a.sa1 + b2 * a.sa2, a.B + b1 * a.sb1 + b2 * a.sb2, (int64_t)tm * T, (int64_t)tn * T};
+  }
+  static VH_DEV int k8_of(bool kc, int u) { return kc ? threadIdx.x & 3 : ((threadIdx.x >> 6) + 4 * u) & 3; }
+  // The pieces of the k tile at k0 of rows r0 .. (R of them, K long) into v.
+  template <bool KC, bool BUF>
+  static VH_DEV void load(const float* X, int64_t ld, int64_t r0, int64_t R, int64_t k0, int64_t K,
+                          vh_f4 (&v)[T / 64][2]);
+  static VH_DEV void load_tile(const GemmArgs& a, const Origin& o, int64_t k0, Regs& R, int set) {
+    load<A_KC, A_BUF>(o.A, a.lda, o.m0, a.M, k0, a.K, R.a[set]);
+    load<B_KC, B_BUF>(o.B, a.ldb, o.n0, a.N, k0, a.K, R.b[set]);
+  }
 };
 
 template <bool A_KC, bool A_BUF, bool B_KC, bool B_BUF, int T>
@@ -283,7 +213,8 @@ VH_DEV void gemm_tile_impl(const GemmArgs& a) {
   } else {
     gm_tile_of(blockIdx.x, gridDim.x, a.tiles_m, a.tiles_n, tm, tn);
   }
-  Tile::run(a, L, tm, tn, bat, (int)blockIdx.y, causal);
+  typename Tile::Regs R;
+  Tile::run(a, L, tm, tn, bat, (int)blockIdx.y, causal, R);
 }
 
 // The persistent form for dense products: the grid is at most the chip's
@@ -297,15 +228,45 @@ VH_DEV void gemm_tile_walk(const GemmArgs& a) {
   for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
     int tm, tn;
     gm_tile_of((int)(it % tiles), tiles, a.tiles_m, a.tiles_n, tm, tn);
-    Tile::run(a, L, tm, tn, it / tiles, (int)(it / tiles), 0);
+    typename Tile::Regs R;
+    Tile::run(a, L, tm, tn, it / tiles, (int)(it / tiles), 0, R);
     __syncthreads();  // the next item stages into the LDS this one read
   }
 }
 
 template <bool A_KC, bool A_BUF, bool B_KC, bool B_BUF, int T>
+template <bool KC, bool BUF>
+VH_DEV void GemmTile<A_KC, A_BUF, B_KC, B_BUF, T>::load(const float* X, int64_t ld, int64_t r0, int64_t R, int64_t k0,
+                                                        int64_t K, vh_f4 (&v)[T / 64][2]) {
+  const uint32_t tid = threadIdx.x, w = tid >> 6, q4 = (tid & 63) >> 4, c4 = tid & 15;
+  if constexpr (BUF) {
+    const auto r = gm_rsrc(X + (KC ? r0 * ld + k0 : k0 * ld + r0),
+                           (KC ? (R - 1 - r0) * ld + K - k0 : (K - 1 - k0) * ld + R - r0) * 4);
+    const uint32_t ld4 = (uint32_t)ld * 4u;
+#pragma unroll
+    for (int u = 0; u < T / 64; ++u) {
+      const uint32_t o = KC ? ((tid >> 2) + 64u * u) * ld4 + k8_of(true, u) * 32u
+                            : (8u * k8_of(false, u) + 2u * q4) * ld4 + (((w + 4u * u) >> 2) * 64u + 4u * c4) * 4u;
+      v[u][0] = gm_bload(r, o);
+      v[u][1] = gm_bload(r, o + (KC ? 16u : ld4));
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < T / 64; ++u)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int64_t r = r0 + (KC ? (tid >> 2) + 64 * u : ((w + 4 * u) >> 2) * 64 + 4 * c4 + (e & 3));
+        const int64_t k = k0 + 8 * k8_of(KC, u) + (KC ? e : 2 * q4 + (e >> 2));
+        v[u][e >> 2][e & 3] = r < R && k < K ? X[KC ? r * ld + k : k * ld + r] : 0.0f;
+      }
+  }
+}
+
+template <bool A_KC, bool A_BUF, bool B_KC, bool B_BUF, int T>
+template <bool STREAM>
 VH_DEV void GemmTile<A_KC, A_BUF, B_KC, B_BUF, T>::run(const GemmArgs& a, Lds& L, int tm, int tn, int64_t bat, int kr,
-                                                       int causal) {
-  static_assert(T == 128 || T == 64, "tile");
+                                                       int causal, Regs& R, const Origin* next) {
+  static_assert((T == 128 || T == 64) && !(STREAM && T == 64), "tile");
   constexpr int NW = T / 64, U = T / 64;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wm = w >> 1, wn = w & 1, li = lane & 31, h = lane >> 5, q4 = lane >> 4, c4 = lane & 15;
@@ -337,44 +298,12 @@ VH_DEV void GemmTile<A_KC, A_BUF, B_KC, B_BUF, T>::run(const GemmArgs& a, Lds& L
   // at k = 2 q and 2 q + 1, and a transpose across the lanes' q leaves it all eight k of
   // row 4 c + q (at LDS piece 16 q + (c + 4 q) % 16 of the block, which the writes and
   // the fragment reads of 16 lanes both meet without bank conflicts).
-  auto k8_of = [&](bool kc, int u) { return kc ? tid & 3 : (w + 4 * u) & 3; };
   auto lds_of = [&](bool kc, int u) {
     const int piece = kc ? (tid >> 2) + 64 * u : ((w + 4 * u) >> 2) * 64 + 16 * q4 + ((c4 + 4 * q4) & 15);
     return k8_of(kc, u) * HS + 4 * piece;
   };
-  vh_f4 ra[D][U][2], rb[D][U][2];
-  // The pieces of the k tile at k0 of rows r0 .. (R of them, K long) into v.
-  auto load = [&](auto kcv, auto bufv, const float* X, int64_t ld, int64_t r0, int64_t R, int64_t k0,
-                  vh_f4 (&v)[U][2]) {
-    constexpr bool KC = decltype(kcv)::value, BUF = decltype(bufv)::value;
-    if constexpr (BUF) {
-      const auto r = gm_rsrc(X + (KC ? r0 * ld + k0 : k0 * ld + r0),
-                             (KC ? (R - 1 - r0) * ld + a.K - k0 : (a.K - 1 - k0) * ld + R - r0) * 4);
-      const uint32_t ld4 = (uint32_t)ld * 4u;
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint32_t o = KC ? ((tid >> 2) + 64u * u) * ld4 + k8_of(true, u) * 32u
-                              : (8u * k8_of(false, u) + 2u * q4) * ld4 + (((w + 4u * u) >> 2) * 64u + 4u * c4) * 4u;
-        v[u][0] = gm_bload(r, o);
-        v[u][1] = gm_bload(r, o + (KC ? 16u : ld4));
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int64_t r = r0 + (KC ? (tid >> 2) + 64 * u : ((w + 4 * u) >> 2) * 64 + 4 * c4 + (e & 3));
-          const int64_t k = k0 + 8 * k8_of(KC, u) + (KC ? e : 2 * q4 + (e >> 2));
-          v[u][e >> 2][e & 3] = r < R && k < a.K ? X[KC ? r * ld + k : k * ld + r] : 0.0f;
-        }
-    }
-  };
   const GmFlag<A_KC> akc{};
   const GmFlag<B_KC> bkc{};
-  auto load_tile = [&](int64_t k0, int set) {
-    load(akc, GmFlag<A_BUF>{}, A, a.lda, m0, a.M, k0, ra[set]);
-    load(bkc, GmFlag<B_BUF>{}, B, a.ldb, n0, a.N, k0, rb[set]);
-  };
   // Factors of the pieces: S3_SCALE, negative in every other group of 32 rows of A and
   // columns of B, and in every other k tile of A: the matrix core's sums drift
   // towards minus infinity by what they round off (gemm_split.h), which then cancels
@@ -453,6 +382,7 @@ VH_DEV void GemmTile<A_KC, A_BUF, B_KC, B_BUF, T>::run(const GemmArgs& a, Lds& L
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(tt[i][j][r], (i ^ j) & 1 ? -sg : sg, acc[i][j][r]);
   };
+  const Origin og{A, B, m0, n0};
   // Loads past the last k tile fetch it again (every load stays in the range).
   auto k_at = [&](int st) { return kb + (int64_t)(st < steps ? st : steps - 1) * GM_TK; };
   if (steps > 0) {
@@ -460,11 +390,11 @@ VH_DEV void GemmTile<A_KC, A_BUF, B_KC, B_BUF, T>::run(const GemmArgs& a, Lds& L
       // Two stages: k tile st is multiplied from one while st + 1 is split into the
       // other (free since the barrier: its readers have passed it), its registers
       // then reloaded with st + 3.
-      load_tile(k_at(0), 0);
-      load_tile(k_at(1), 1);
-      stage(akc, ra[0], L[0][0], k_at(0), fsa * k_sign(kb));
-      stage(bkc, rb[0], L[0][1], k_at(0), fsb);
-      load_tile(k_at(2), 0);
+      load_tile(a, og, k_at(0), R, 0);
+      load_tile(a, og, k_at(1), R, 1);
+      stage(akc, R.a[0], L[0][0], k_at(0), fsa * k_sign(kb));
+      stage(bkc, R.b[0], L[0][1], k_at(0), fsb);
+      load_tile(a, og, k_at(2), R, 0);
       for (int st = 0; st < steps; st += 2) {
 #pragma unroll
         for (int d = 0; d < 2; ++d) {
@@ -473,20 +403,23 @@ VH_DEV void GemmTile<A_KC, A_BUF, B_KC, B_BUF, T>::run(const GemmArgs& a, Lds& L
             frags(L[d][0], L[d][1], 0);
             frags(L[d][0], L[d][1], 1);
             products(0);
-            stage(akc, ra[d ^ 1], L[d ^ 1][0], k_at(st + d + 1), fsa * k_sign(k_at(st + d + 1)));
+            stage(akc, R.a[d ^ 1], L[d ^ 1][0], k_at(st + d + 1), fsa * k_sign(k_at(st + d + 1)));
             products(1);
-            stage(bkc, rb[d ^ 1], L[d ^ 1][1], k_at(st + d + 1), fsb);
-            load_tile(k_at(st + d + 3), d ^ 1);
+            stage(bkc, R.b[d ^ 1], L[d ^ 1][1], k_at(st + d + 1), fsb);
+            load_tile(a, og, k_at(st + d + 3), R, d ^ 1);
             add(k_sign(k_at(st + d)));
           }
         }
       }
     } else {
-      load_tile(k_at(0), 0);
+      if constexpr (!STREAM) load_tile(a, og, k_at(0), R, 0);
       for (int st = 0; st < steps; ++st) {
-        stage(akc, ra[0], L[0][0], k_at(st), fsa * k_sign(k_at(st)));
-        stage(bkc, rb[0], L[0][1], k_at(st), fsb);
-        load_tile(k_at(st + 1), 0);
+        stage(akc, R.a[0], L[0][0], k_at(st), fsa * k_sign(k_at(st)));
+        stage(bkc, R.b[0], L[0][1], k_at(st), fsb);
+        if (STREAM && next && st + 1 == steps)
+          load_tile(a, *next, 0, R, 0);
+        else
+          load_tile(a, og, k_at(st + 1), R, 0);
         lds_barrier();
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
@@ -529,29 +462,32 @@ VH_DEV void GemmTile<A_KC, A_BUF, B_KC, B_BUF, T>::run(const GemmArgs& a, Lds& L
   float* out = split ? a.ws + (int64_t)kr * a.M * a.N : C;
   const float* E0 = gm_addend(a);
   const float* E = !split && E0 ? E0 + b1 * a.se1 + b2 * a.se2 : nullptr;
-  gm_store_direct<NW, NW>(a, acc, out, split ? a.N : a.ldc, E, split, m0, n0, T, wm, wn, li, h);
+  gm_store_direct<NW, NW, STREAM>(a, acc, out, split ? a.N : a.ldc, E, split, m0, n0, T, wm, wn, li, h);
 }
 
 // Persistent form for batched products with a short k range (attention's
 // scores q k^T and dP = dO v^T: K = Dk = 64, 2 k tiles per C tile). Launched
 // as one workgroup per resident slot (a multiple of 8), each walks a list of
-// C tiles as one continuous k loop: the last k step of a tile loads the
+// 128 x 128 C tiles as one continuous k loop: the last k step of a tile loads the
 // first k tile of the next one, so its global loads are in flight under the
 // current tile's products and epilogue instead of exposed at the start of a
 // short-lived workgroup. Work items are the live tiles of every batch, batch
 // major (causal 1: the tiles with tn <= tm, which with tiles_n >= tiles_m are
 // T (T + 1) / 2 for T = tiles_m); XCD x (= workgroup id % 8, the hardware's
 // round-robin) takes the x-th contiguous eighth of the items, so one XCD works
-// on one or two batches at a time and its L2 holds their operands. Tile width
-// 128; no split, causal 0 or 1 only (the host guarantees both).
-template <bool A_KC, bool A_VEC, bool B_KC, bool B_VEC>
-VH_DEV void gemm_f32_persist(const GemmArgs& a) {
-  constexpr int TN = 128, NTW = 2;
-  __shared__ __attribute__((aligned(16))) float L[4][GM_STAGE];  // A stages 0-1, B stages 2-3
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wm = w >> 1, wn = w & 1, li = lane & 31, h = lane >> 5;
+// on one or two batches at a time and its L2 holds their operands. No split,
+// causal 0 or 1 only (the host guarantees both).
+//
+// 192 x [1024, 64] x [64, 1024], causal (453 MB of live tiles): 172 us on the f32
+// instruction (92 us of it matrix work at that instruction's peak), 150 on the
+// three-part split, 3.0 TB/s written. The instruction's rate no longer bounds it:
+// the splits, LDS traffic and stores of each 64-deep tile do, two workgroups per
+// CU (registers) covering each other's.
+template <bool A_KC, bool B_KC>
+VH_DEV void gemm_tile_stream(const GemmArgs& a) {
+  using Tile = GemmTile<A_KC, true, B_KC, true, 128>;
+  __shared__ __attribute__((aligned(1024))) typename Tile::Lds L;
   const int causal = gm_causal(a);
-  const float* E0 = gm_addend(a);
   const int64_t live = causal == 1 ? (int64_t)a.tiles_m * (a.tiles_m + 1) / 2 : (int64_t)a.tiles_m * a.tiles_n;
   const int64_t total = live * a.nbat;
   const int nloc = (int)(gridDim.x / 8), x = (int)(blockIdx.x % 8);
@@ -560,127 +496,38 @@ VH_DEV void gemm_f32_persist(const GemmArgs& a) {
   int64_t item = x * per + (int64_t)(blockIdx.x / 8);
   if (item >= end) return;
 
-  struct Tile {
-    const float* A;
-    const float* B;
-    float* C;
-    const float* E;
-    int64_t m0, n0;
-    bool inside;  // the whole tile and its k range are inside A, B and C
-  };
-  auto decode = [&](int64_t it, Tile& t) {
-    const int64_t bat = it / live;
+  auto decode = [&](int64_t it, int& tm, int& tn, int64_t& bat) {
+    bat = it / live;
     const int64_t u = it % live;
-    int64_t tm, tn;
     if (causal == 1) {  // u = tm (tm + 1) / 2 + tn, tn <= tm
-      tm = (int64_t)((sqrtf(8.0f * (float)u + 1.0f) - 1.0f) * 0.5f);
-      while (tm * (tm + 1) / 2 > u) --tm;
-      while ((tm + 1) * (tm + 2) / 2 <= u) ++tm;
-      tn = u - tm * (tm + 1) / 2;
+      int64_t t = (int64_t)((sqrtf(8.0f * (float)u + 1.0f) - 1.0f) * 0.5f);
+      while (t * (t + 1) / 2 > u) --t;
+      while ((t + 1) * (t + 2) / 2 <= u) ++t;
+      tm = (int)t;
+      tn = (int)(u - t * (t + 1) / 2);
     } else {
-      tm = u / a.tiles_n;
-      tn = u % a.tiles_n;
+      tm = (int)(u / a.tiles_n);
+      tn = (int)(u % a.tiles_n);
     }
-    const int64_t b1 = bat / a.nb2, b2 = bat % a.nb2;
-    t.A = a.A + b1 * a.sa1 + b2 * a.sa2;
-    t.B = a.B + b1 * a.sb1 + b2 * a.sb2;
-    t.C = a.C + b1 * a.sc1 + b2 * a.sc2;
-    t.E = E0 ? E0 + b1 * a.se1 + b2 * a.se2 : nullptr;
-    t.m0 = tm * GM_TM;
-    t.n0 = tn * TN;
-    t.inside = t.m0 + GM_TM <= a.M && t.n0 + TN <= a.N && a.K % GM_TK == 0;
   };
-
-  Tile cur, nxt;
-  decode(item, cur);
-  float sa[GM_TM / 8], sb[TN / 8];
-  gm_load<A_KC, A_VEC, GM_TM>(cur.A, a.lda, cur.m0, a.M, 0, a.K, tid, sa);
-  gm_load<B_KC, B_VEC, TN>(cur.B, a.ldb, cur.n0, a.N, 0, a.K, tid, sb);
-  gm_store_lds<A_KC, A_VEC, GM_TM>(L[0], tid, sa);
-  gm_store_lds<B_KC, B_VEC, TN>(L[2], tid, sb);
-  __syncthreads();
-  int s = 0;
-
-  constexpr int RD = 4 * ((A_KC ? 2 : 8) + NTW * (B_KC ? 1 : 4));
-  constexpr int WR = (A_VEC ? GM_TM / 32 : GM_TM / 8) + (B_VEC ? TN / 32 : TN / 8);
-  constexpr int VM = WR;
-  constexpr int MF = 8 * NTW;
+  int tm, tn;
+  int64_t bat;
+  decode(item, tm, tn, bat);
+  typename Tile::Regs R;
+  Tile::load_tile(a, Tile::origin(a, tm, tn, bat), 0, R, 0);
   for (;;) {
     const int64_t nit = item + nloc;
-    const bool has_next = nit < end;
-    if (has_next)
-      decode(nit, nxt);
-    else
-      nxt = cur;
-    vh_f32x16 acc[2][NTW];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < NTW; ++j) acc[i][j] = vh_f32x16{};
-    // One k step: the next stage (this tile's next k tile, else the next
-    // tile's first, else this one's last again) is loaded, this stage is
-    // multiplied, and the loaded one is staged into the other LDS buffer.
-    auto k_loop = [&](auto unchecked) {
-      constexpr bool CHECK = !decltype(unchecked)::value;
-      for (int64_t k0 = 0; k0 < a.K; k0 += GM_TK) {
-        const bool more = k0 + GM_TK < a.K;
-        const float* An = more ? cur.A : nxt.A;
-        const float* Bn = more ? cur.B : nxt.B;
-        const int64_t mn = more ? cur.m0 : nxt.m0, nn = more ? cur.n0 : nxt.n0;
-        const int64_t kn = more ? k0 + GM_TK : (has_next ? 0 : k0);
-        if constexpr (CHECK) {
-          if (more || has_next) {
-            gm_load<A_KC, A_VEC, GM_TM>(An, a.lda, mn, a.M, kn, a.K, tid, sa);
-            gm_load<B_KC, B_VEC, TN>(Bn, a.ldb, nn, a.N, kn, a.K, tid, sb);
-          }
-        } else {
-          gm_load<A_KC, A_VEC, GM_TM, false>(An, a.lda, mn, a.M, kn, a.K, tid, sa);
-          gm_load<B_KC, B_VEC, TN, false>(Bn, a.ldb, nn, a.N, kn, a.K, tid, sb);
-        }
-        vh_f4 fa[4][2], fb[4][NTW];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int kc = h * 16 + 4 * q;
-          fa[q][0] = gm_frag<A_KC>(L[s], wm * 64 + li, kc);
-          fa[q][1] = gm_frag<A_KC>(L[s], wm * 64 + 32 + li, kc);
-#pragma unroll
-          for (int nt = 0; nt < NTW; ++nt) fb[q][nt] = gm_frag<B_KC>(L[2 + s], wn * (TN / 2) + nt * 32 + li, kc);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-#pragma unroll
-            for (int nt = 0; nt < NTW; ++nt) {
-              acc[0][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][0][e], fb[q][nt][e], acc[0][nt], 0, 0, 0);
-              acc[1][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q][1][e], fb[q][nt][e], acc[1][nt], 0, 0, 0);
-            }
-          }
-        }
-        gm_store_lds<A_KC, A_VEC, GM_TM>(L[s ^ 1], tid, sa);
-        gm_store_lds<B_KC, B_VEC, TN>(L[2 + (s ^ 1)], tid, sb);
-        if constexpr (!CHECK) __builtin_amdgcn_sched_group_barrier(0x020, VM, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, RD, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 3 * MF, 0);
-#pragma unroll
-        for (int i = 0; i < MF; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x200, (WR + MF - 1) / MF, 0);
-        }
-        __syncthreads();
-        s ^= 1;
-      }
-    };
-    if (cur.inside && nxt.inside)
-      k_loop(GmFlag<true>{});
-    else
-      k_loop(GmFlag<false>{});
-    // Streaming stores: with normal ones the write of a score-sized output
-    // runs at ~1.8 TB/s here, with these at ~2.8 TB/s (measured).
-    gm_store_direct<2, NTW, true>(a, acc, cur.C, a.ldc, cur.E, false, cur.m0, cur.n0, GM_TM, wm, wn, li, h);
-    if (!has_next) break;
+    const bool more = nit < end;
+    int tm2 = tm, tn2 = tn;
+    int64_t bat2 = bat;
+    if (more) decode(nit, tm2, tn2, bat2);
+    const typename Tile::Origin next = Tile::origin(a, tm2, tn2, bat2);
+    Tile::template run<true>(a, L, tm, tn, bat, 0, causal, R, &next);
+    if (!more) break;
     item = nit;
-    cur = nxt;
+    tm = tm2;
+    tn = tn2;
+    bat = bat2;
   }
 }
 

@@ -252,9 +252,9 @@ K_GEMMT(true, true, vh_gemmt_kk)
 K_GEMMT(true, false, vh_gemmt_kn)
 K_GEMMT(false, true, vh_gemmt_mk)
 K_GEMMT(false, false, vh_gemmt_mn)
-// Persistent form of the 128-bit-load layouts (batched products with short k).
+// 128 x 128 tiles as one stream of k tiles (batched products with short k).
 #define K_GEMMP(AK, BK, NAME) \
-  extern "C" __global__ void __launch_bounds__(256, 2) NAME(GemmArgs a) { gemm_f32_persist<AK, true, BK, true>(a); }
+  extern "C" __global__ void __launch_bounds__(256, 2) NAME(GemmArgs a) { gemm_tile_stream<AK, BK>(a); }
 K_GEMMP(true, true, vh_gemmp_k4_k4)
 K_GEMMP(true, false, vh_gemmp_k4_n4)
 K_GEMMP(false, true, vh_gemmp_m4_k4)
