@@ -86,6 +86,7 @@ SIGNATURES = {
     "vh_last_error": (ctypes.c_char_p, []),
     "vh_stream": (c_void_p, []),
     "vh_gemm_last_path": (c_int, []),
+    "vh_gemm_last_kernel": (ctypes.c_char_p, []),
     "vh_device_cu_count": (c_int, []),
     "vh_sync": (c_int, []),
     "vh_check_device_error": (c_int, []),

@@ -1458,6 +1458,13 @@ GemmArgs gemm_args(const vh_gemm_desc* d, int64_t lda, int64_t ldb, int64_t tile
 
 namespace {
 thread_local int g_gemm_path = VH_GEMM_PATH_NONE;
+thread_local char g_gemm_kernel[32] = "";  // vh_gemm_last_kernel's name
+
+// launch() of a product kernel, noted for vh_gemm_last_kernel.
+int launch_product(const std::string& name, int64_t gx, int64_t gy, unsigned block, hipStream_t s, const GemmArgs& g) {
+  std::snprintf(g_gemm_kernel, sizeof g_gemm_kernel, "%s", name.c_str());
+  return launch(name, gx, gy, block, 0, s, g);
+}
 
 // How the persistent kernel (kernels/gemm_split.h) runs a product: tile width and
 // whether the last, partly filled round of tiles is split along K over all
@@ -1521,7 +1528,7 @@ int gemm_split_k(const vh_gemm_desc* d, const GemmPlan& plan, int64_t lda, int64
   g.ksplit = (int32_t)ks;
   g.kchunk = plan.kchunk;
   g.ws = static_cast<float*>(ws);
-  int rc = launch(name, gx, gy, 256, 0, s, g);
+  int rc = launch_product(name, gx, gy, 256, s, g);
   if (rc == VH_OK) {
     GemmReduceArgs r{g.ws, d->c, d->e, M, N, d->c_sm, d->e_sm, d->e_sn, (int32_t)ks, d->accumulate ? 1 : 0, d->alpha};
     rc = launch("vh_gemm_reduce", std::min<int64_t>(cdiv(M * N, 256), 8192), 1, 256, 0, s, r);
@@ -1539,7 +1546,7 @@ int gemm_walk(const vh_gemm_desc* d, const GemmPlan& plan, bool akc, bool bkc, i
   if (plan.ksplit > 1) return gemm_split_k(d, plan, lda, ldb, name, grid, 1, s);
   GemmArgs g = gemm_args(d, lda, ldb, tiles_m, tiles_n);
   g.nbat = nb;
-  return launch(name, grid, 1, 256, 0, s, g);
+  return launch_product(name, grid, 1, 256, s, g);
 }
 
 // One launch of the split persistent kernel (and its fix-up).
@@ -1557,7 +1564,7 @@ int gemm_split_range(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int
     g.ws = static_cast<float*>(ws);
   }
   const std::string bn = std::to_string(plan.bn);
-  int rc = launch(std::string("vh_gemms_") + (akc ? "k" : "m") + (bkc ? "k" : "n") + "_" + bn, G, 1, 512, 0, s, g);
+  int rc = launch_product(std::string("vh_gemms_") + (akc ? "k" : "m") + (bkc ? "k" : "n") + "_" + bn, G, 1, 512, s, g);
   if (rc == VH_OK && ws) {
     GemmArgs x = g;
     x.ksplit = G;
@@ -1641,7 +1648,7 @@ int gemm_big(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t ldb
   }
   const std::string bn = std::to_string(BN);
   const std::string name = std::string("vh_gemmb_") + (akc ? "k" : "m") + (bkc ? "k" : "n") + "_" + bn;
-  int rc = launch(name, G, 1, 512, 0, s, g);
+  int rc = launch_product(name, G, 1, 512, s, g);
   if (rc == VH_OK && rem > 0) {
     GemmArgs f = g;
     f.ksplit = G;
@@ -1660,6 +1667,7 @@ int gemm_big(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t ldb
     t.accumulate = 1;
     t.engine = VH_GEMM_ENGINE_TILED;
     VH_TRY(vh_gemm(&t, s));
+    std::snprintf(g_gemm_kernel, sizeof g_gemm_kernel, "%s", name.c_str());
   }
   g_gemm_path = VH_GEMM_PATH_PERSISTENT;
   return VH_OK;
@@ -1667,9 +1675,11 @@ int gemm_big(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t ldb
 }  // namespace
 
 int vh_gemm_last_path(void) { return g_gemm_path; }
+const char* vh_gemm_last_kernel(void) { return g_gemm_kernel; }
 
 int vh_gemm(const vh_gemm_desc* d, void* stream) {
   g_gemm_path = VH_GEMM_PATH_NONE;
+  g_gemm_kernel[0] = '\0';
   VH_TRY(require_init());
   if (!d) return fail(VH_ERR_INVALID, "vh_gemm: null descriptor");
   const int64_t M = d->M, N = d->N, K = d->K;
@@ -1749,7 +1759,7 @@ int vh_gemm(const vh_gemm_desc* d, void* stream) {
     GemmArgs g = gemm_args(d, lda, ldb, pm, pn);
     g.nbat = nbat;
     const std::string pname = std::string("vh_gemmp_") + (akc ? "k4" : "m4") + "_" + (bkc ? "k4" : "n4");
-    VH_TRY(launch(pname, slots, 1, 256, 0, s, g));
+    VH_TRY(launch_product(pname, slots, 1, 256, s, g));
     g_gemm_path = VH_GEMM_PATH_BATCHED;
     return VH_OK;
   }
@@ -1759,7 +1769,7 @@ int vh_gemm(const vh_gemm_desc* d, void* stream) {
   for (int64_t b0 = 0; b0 < d->batch[0]; b0 += outer_chunk) {
     const int64_t nb = std::min(outer_chunk, d->batch[0] - b0);
     const GemmArgs g = gemm_args(d, lda, ldb, tiles_m, tiles_n, b0);
-    VH_TRY(launch(name, (tiles_m * tiles_n), (nb * d->batch[1]), 256, 0, s, g));
+    VH_TRY(launch_product(name, (tiles_m * tiles_n), (nb * d->batch[1]), 256, s, g));
   }
   g_gemm_path = VH_GEMM_PATH_TILED;
   return VH_OK;
