@@ -1589,18 +1589,24 @@ int gemm_split(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t l
   if (!gemm_persistent_ok(d, lda, ldb)) return VH_OK;
   // Below ~1e9 multiply-adds the 256-row tiles are too few or their pieces too many:
   // the 64 x 64 tiles where their estimate is less ([1000, 768] x [768, 768]: 36.7 us
-  // with its fix-up against 22.3; 5 us of launches are added to the other's).
+  // with its fix-up against 22.3; 5 us of launches are added to the other's). K <= 2
+  // never runs on the 256-row tiles: gemm.h has the f32 instruction there, which is
+  // more exact (2-norm error K = 1 2.53e-8 against the split's 3.44e-8, K = 2 3.11e-8
+  // against 3.36e-8, and 2.0 u against 2.8 u of sum |a b| at most; K = 3 3.60e-8 against
+  // 3.29e-8, 4 3.98e-8 against 3.24e-8).
   const int64_t nb = d->batch[0] * d->batch[1];
+  const bool tiny = d->K <= 2;
   if (d->K <= 16384 && (double)cdiv(d->M, 64) * (double)cdiv(d->N, 64) * (double)nb < 1e6) {
     const GemmPlan tiled = gemm_plan(d->M, d->N, d->K, nb, nb == 1);
     const int G = std::max(8, g_rt.cu_count / 8 * 8);
-    if (tiled.tile == 64 && tiled.us < gemm_split_plan(d->M, d->N, d->K, nb, G).us + 5.0) {
+    if (tiled.tile == 64 && (tiny || tiled.us < gemm_split_plan(d->M, d->N, d->K, nb, G).us + 5.0)) {
       VH_TRY(gemm_walk(d, tiled, akc, bkc, lda, ldb, s));
       *taken = true;
       g_gemm_path = VH_GEMM_PATH_PERSISTENT;
       return VH_OK;
     }
   }
+  if (tiny) return VH_OK;
   const int64_t K = d->K, n = K > 16384 ? cdiv(K, 8192) : 1;
   const int64_t kc = cdiv(cdiv(K, n), VH_GEMMS_TK) * VH_GEMMS_TK;
   for (int64_t k0 = 0; k0 < K; k0 += kc) {
