@@ -488,11 +488,6 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
       // Whole tile inside C with a full addend E[m, n]: v = alpha acc + E
       // (+ old C), in gm_finish's order, without bounds tests.
       float* base = Cb + (cur.m0 + lrow) * ldo + cur.n0 + lcol;
-      const float* E = Eb;
-      const bool ecol = E && a.sem == 0;
-      float eb[NB];
-#pragma unroll
-      for (int jj = 0; jj < NB; ++jj) eb[jj] = ecol ? E[(cur.n0 + lcol + 32 * jj) * a.sen] : 0.0f;
 #pragma unroll
       for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -502,10 +497,7 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
 #pragma unroll
           for (int jj = 0; jj < NB; ++jj) {
             float v = acc[i][jj][r] * a.alpha;
-            if (ecol)
-              v = v + eb[jj];
-            else if (E)
-              v = v + E[(cur.m0 + lrow + rl) * a.sem + (cur.n0 + lcol + 32 * jj) * a.sen];
+            v = v + Eb[(cur.m0 + lrow + rl) * a.sem + (cur.n0 + lcol + 32 * jj) * a.sen];
             if (a.accumulate) v = row[32 * jj] + v;
             row[32 * jj] = v;
           }
