@@ -8,7 +8,10 @@
 // range) segments as one continuous stream of k tiles, whole-tile rounds and a
 // last round that is split along K over all workgroups or left whole
 // (a.whole_tail), a fix-up adding the pieces in k order. Here any K runs in
-// whole: the last k tile is masked in LDS.
+// whole: the last k tile is masked in LDS. A tile of a round left whole may be summed
+// in several chains of k tiles (a.whole_tail of them), each added to C by the thread
+// that stored the ones before: the host asks for it where one chain would round
+// more than the pieces of a split round (gemm_split_plan).
 //
 // What bounds it: the chip's power. On MI355X the matrix cores hold 2.4 GHz on
 // zeros (lm_head dx [16384, 50272] x [50272, 768]: 3.86 ms, 328 TFLOP/s of f32
@@ -96,15 +99,21 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
   // takes G / 8 consecutive tiles, or its eighth of an unsplit last round.
   const int x = g % 8, local = x * (G / 8) + g / 8;
   const int xlo = sp.rem * x / 8, xn = sp.rem * (x + 1) / 8 - xlo;
-  const int ndp = sp.full + (a.whole_tail && g / 8 < xn ? 1 : 0);  // whole-tile segments
+  const int nch = a.whole_tail > 1 ? a.whole_tail : 1;  // chains per whole tile
+  const int ndp = (sp.full + (a.whole_tail && g / 8 < xn ? 1 : 0)) * nch;  // whole-tile segments
   const int nseg = ndp + npieces;
   if (nseg == 0) return;
   auto seg_of = [&](int j) {
     GbSeg s;
     int u, kt0 = 0, kt1 = sp.nk;
     s.slot = -1;
+    s.more = false;
     if (j < ndp) {
-      u = j * G + (j < sp.full ? local : xlo + g / 8);
+      const int t = j / nch, c = j - t * nch;
+      u = t * G + (t < sp.full ? local : xlo + g / 8);
+      kt0 = sp.nk * c / nch;  // (the host keeps nk * nch below 2^31)
+      kt1 = sp.nk * (c + 1) / nch;
+      s.more = c > 0;
     } else {
       const int p = j - ndp, t = t0 + p;  // (never with whole_tail)
       u = sp.full * G + t;
@@ -422,10 +431,13 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
         }
       return;
     }
+    using T = std::true_type;
+    using F = std::false_type;
     const bool inner = cur.m0 + GB_TM <= a.M && cur.n0 + BN <= a.N;
     float* const Cb = a.C + cur.co;
-    const float* const Eb = a.E ? a.E + cur.eo : nullptr;
-    if (inner && !a.E && !a.accumulate) {
+    const float* const Eb = a.E && !cur.more ? a.E + cur.eo : nullptr;
+    const bool accumulate = a.accumulate || cur.more;
+    if (inner && !Eb && !accumulate) {
       float* base = Cb + (cur.m0 + lrow) * ldo + cur.n0 + lcol;
 #pragma unroll
       for (int i = 0; i < WM; ++i)
@@ -475,10 +487,8 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
             }
           }
       };
-      using T = std::true_type;
-      using F = std::false_type;
       if (Eb) {
-        if (a.accumulate) tile(T{}, T{}); else tile(T{}, F{});
+        if (accumulate) tile(T{}, T{}); else tile(T{}, F{});
       } else {
         tile(F{}, T{});  // accumulate (the plain store returned above)
       }
@@ -498,27 +508,73 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
           for (int jj = 0; jj < NB; ++jj) {
             float v = acc[i][jj][r] * a.alpha;
             v = v + Eb[(cur.m0 + lrow + rl) * a.sem + (cur.n0 + lcol + 32 * jj) * a.sen];
-            if (a.accumulate) v = row[32 * jj] + v;
+            if (accumulate) v = row[32 * jj] + v;
             row[32 * jj] = v;
           }
         }
       return;
     }
+    // A tile at an edge of C: rows below mlim and columns below nlim of this lane's. The
+    // reads of old C again go out 8 rows x NB columns at a time, and are waited for once:
+    // under per-element tests the compiler would wait for everything at each element.
+    const int64_t mr = a.M - cur.m0 - lrow, nr = a.N - cur.n0 - lcol;
+    int mlim = mr < GB_TM ? (int)mr : GB_TM, nlim = nr < BN ? (int)nr : BN;
+    float* base = Cb + (cur.m0 + lrow) * ldo + cur.n0 + lcol;
+    if (Eb && a.sem != 0) {  // a full addend
 #pragma unroll
-    for (int i = 0; i < WM; ++i)
-#pragma unroll
-      for (int jj = 0; jj < NB; ++jj) {
-        const int64_t n = cur.n0 + lcol + 32 * jj;
+      for (int i = 0; i < WM; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
+          asm volatile("" : "+v"(mlim), "+v"(nlim));  // (tests and offsets formed here, as above)
           const int rl = 32 * i + 8 * (r >> 2) + (r & 3);
-          const int64_t m = cur.m0 + lrow + rl;
-          if (m < a.M && n < a.N) {
-            float* cp = Cb + m * ldo + n;
-            *cp = gm_finish(a, Eb, false, acc[i][jj][r], m, n, a.accumulate ? *cp : 0.0f);
-          }
+#pragma unroll
+          for (int jj = 0; jj < NB; ++jj)
+            if (rl < mlim && 32 * jj < nlim) {
+              float v = acc[i][jj][r] * a.alpha;
+              v = v + Eb[(cur.m0 + lrow + rl) * a.sem + (cur.n0 + lcol + 32 * jj) * a.sen];
+              if (accumulate) v = base[rl * ldo + 32 * jj] + v;
+              base[rl * ldo + 32 * jj] = v;
+            }
         }
-      }
+      return;
+    }
+    float eb[NB];
+#pragma unroll
+    for (int jj = 0; jj < NB; ++jj) eb[jj] = Eb && 32 * jj < nlim ? Eb[(cur.n0 + lcol + 32 * jj) * a.sen] : 0.0f;
+    auto edge = [&](auto has_bias, auto acc_c) {
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int r0 = 0; r0 < 16; r0 += 8) {
+          asm volatile("" : "+v"(mlim), "+v"(nlim));
+          float old[8][NB];
+          if constexpr (decltype(acc_c)::value) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r)
+#pragma unroll
+              for (int jj = 0; jj < NB; ++jj) {
+                const int rl = 32 * i + 8 * ((r0 + r) >> 2) + ((r0 + r) & 3);
+                old[r][jj] = rl < mlim && 32 * jj < nlim ? base[rl * ldo + 32 * jj] : 0.0f;
+              }
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+          }
+#pragma unroll
+          for (int r = 0; r < 8; ++r)
+#pragma unroll
+            for (int jj = 0; jj < NB; ++jj) {
+              const int rl = 32 * i + 8 * ((r0 + r) >> 2) + ((r0 + r) & 3);
+              float v = acc[i][jj][r0 + r] * a.alpha;  // (gm_finish's order)
+              if constexpr (decltype(has_bias)::value) v = v + eb[jj];
+              if constexpr (decltype(acc_c)::value) v = old[r][jj] + v;
+              if (rl < mlim && 32 * jj < nlim) base[rl * ldo + 32 * jj] = v;
+            }
+        }
+    };
+    if (Eb) {
+      if (accumulate) edge(T{}, T{}); else edge(T{}, F{});
+    } else {
+      if (accumulate) edge(F{}, T{}); else edge(F{}, F{});
+    }
   };
   // Segments in order; per segment, one k step per k tile on alternating
   // stages (the staged tile -- the next in the stream -- goes to LDS and the

@@ -1471,7 +1471,7 @@ int launch_product(const std::string& name, int64_t gx, int64_t gy, unsigned blo
 // workgroups (stream-K) or run as it is on as many workgroups as it has tiles.
 struct SplitPlan {
   int64_t bn;
-  bool whole_tail;
+  int whole_tail;  // 0: split; n: unsplit, n chains per sum
   double us;  // the estimate the choice was made by
 };
 
@@ -1486,16 +1486,26 @@ struct SplitPlan {
 // 768 (192 / 256 tiles): K = 768 99 / 94, K = 3072 367 / 349 us, K = 50272 5.82 /
 // 5.63 ms. Split / unsplit at 256 wide: 192 tiles of 48 k tiles 138 / 99 us, of 192
 // 388 / 363, of 3142 5.81 / 6.01 ms; 64 tiles of 48 296 / 310 us; 9 of 1024 118 / 1640.
-SplitPlan gemm_split_plan(int64_t M, int64_t N, int64_t K, int64_t nb, int G) {
-  SplitPlan best{0, false, 0.0};
+//
+// Chains. A sum over K rounds about 0.85 as much as on the f32 instruction
+// (split3.h), whose kernel splits every partly filled round: t 256 x 192 tiles short
+// of one round are cut into some G / t chains each, and one chain of them all would
+// be less exact ([7000, 768] x [768, 768], t = 112: 4.14e-7 against 3.09e-7). A round
+// left whole is then summed in as many chains, at ~9 us (256 wide) for each further one.
+// `ranges`: the launches that K itself is cut into (gemm_split).
+SplitPlan gemm_split_plan(int64_t M, int64_t N, int64_t K, int64_t nb, int G, int64_t ranges = 1) {
+  SplitPlan best{0, 0, 0.0};
   const double nk = (double)cdiv(K, VH_GEMMS_TK);
+  const int64_t narrow = cdiv(M, VH_GEMMB_TM) * cdiv(N, VH_GEMMB_TN) * nb;
+  const int64_t chains = std::max<int64_t>(1, std::min(cdiv(cdiv(G, narrow), ranges), K / 32));
   for (int64_t bn : {VH_GEMMB_TN_WIDE, VH_GEMMB_TN}) {
     const double share = bn == VH_GEMMB_TN_WIDE ? 1.0 : 0.75, step = bn == VH_GEMMB_TN_WIDE ? 2.40 : 1.82;
     const int64_t tiles = cdiv(M, VH_GEMMB_TM) * cdiv(N, bn) * nb, rem = tiles % G;
-    const double whole = nk * std::max(1.4 * share - step * (double)rem / G, 0.09 * share);
+    const double whole =
+        nk * std::max(1.4 * share - step * (double)rem / G, 0.09 * share) + 9.0 * share * (double)(chains - 1);
     const double split = 5.0 + 0.1 * share * (double)(G + rem);
     const double us = nk * step * (double)tiles / G + (rem ? std::min(whole, split) : 0.0);
-    if (!best.bn || us < best.us) best = SplitPlan{bn, rem > 0 && whole < split, us};
+    if (!best.bn || us < best.us) best = SplitPlan{bn, rem > 0 && whole < split ? (int)chains : 0, us};
   }
   return best;
 }
@@ -1550,14 +1560,14 @@ int gemm_walk(const vh_gemm_desc* d, const GemmPlan& plan, bool akc, bool bkc, i
 }
 
 // One launch of the split persistent kernel (and its fix-up).
-int gemm_split_range(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t ldb, hipStream_t s) {
+int gemm_split_range(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t ldb, int64_t ranges, hipStream_t s) {
   const int64_t M = d->M, N = d->N, K = d->K, nb = d->batch[0] * d->batch[1];
   const int G = std::max(8, g_rt.cu_count / 8 * 8);
-  const SplitPlan plan = gemm_split_plan(M, N, K, nb, G);
+  const SplitPlan plan = gemm_split_plan(M, N, K, nb, G, ranges);
   const int64_t tiles_m = cdiv(M, VH_GEMMB_TM), tiles_n = cdiv(N, plan.bn), rem = tiles_m * tiles_n * nb % G;
   GemmArgs g = gemm_args(d, lda, ldb, tiles_m, tiles_n);
   g.nbat = nb;
-  g.whole_tail = plan.whole_tail ? 1 : 0;
+  g.whole_tail = plan.whole_tail;
   void* ws = nullptr;
   if (rem > 0 && !plan.whole_tail) {
     VH_TRY(g_arena.alloc((size_t)(G * VH_GEMMB_SLOTS * VH_GEMMB_TM * plan.bn) * sizeof(float), s, &ws));
@@ -1618,7 +1628,7 @@ int gemm_split(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t l
       t.e = nullptr;
       t.accumulate = 1;
     }
-    VH_TRY(gemm_split_range(&t, akc, bkc, lda, ldb, s));
+    VH_TRY(gemm_split_range(&t, akc, bkc, lda, ldb, n, s));
   }
   *taken = true;
   g_gemm_path = VH_GEMM_PATH_PERSISTENT;

@@ -128,7 +128,7 @@ struct GemmArgs {
   float* ws;
   int64_t nbat;  // persistent form (vh_gemmp_*): batches in the launch (grid y is 1)
   const int32_t* causal_flag;  // non-null: `causal` applies only when *causal_flag is 1, else dense
-  int32_t whole_tail;          // vh_gemms_*: 1 leaves the last round's tiles unsplit
+  int32_t whole_tail;          // vh_gemms_*: n > 0 leaves the last round's tiles unsplit, each sum in n chains over K
   int32_t fix_rows;            // vh_gemm[bs]_fix_*: tile rows per workgroup (divides 256)
 };
 
