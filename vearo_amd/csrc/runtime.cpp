@@ -1477,15 +1477,16 @@ struct SplitPlan {
 
 // Estimated time of each form. The kernel is bound by the chip's power, not by
 // its clock limit: measured on MI355X, a k step takes 2.40 us (256 wide) or 1.82
-// us (192 wide: 1 % more per column) with all 256 workgroups busy, in proportion
-// to how many are, but no less than 1.4 / 1.05 us (2.4 GHz). So an unsplit round
-// on a share f of the chip loses max(1.4 - 2.4 f, 0.09) us per k tile, while a
-// split one writes and reads back a 256 KB (192 KB) piece per workgroup and tile,
-// ~0.1 us each, plus the fix-up's launch. Measured, 256 / 192 wide: N = 50272 over
-// K = 768 5.71 / 5.99 ms; N = 3072 345 / 364 us; N = 2304 (2.25 / 3 rounds) 286 / 273; N =
-// 768 (192 / 256 tiles): K = 768 99 / 94, K = 3072 367 / 349 us, K = 50272 5.82 /
-// 5.63 ms. Split / unsplit at 256 wide: 192 tiles of 48 k tiles 138 / 99 us, of 192
-// 388 / 363, of 3142 5.81 / 6.01 ms; 64 tiles of 48 296 / 310 us; 9 of 1024 118 / 1640.
+// us (192 wide: 1 % more per column) with all 256 workgroups busy; in a round left
+// whole on a share f of them 0.77 + 1.63 f (0.62 + 1.24 f), no less than 1.6 (1.3), where
+// a split round takes its share of the full step but writes and reads back a
+// 256 KB (192 KB) piece per workgroup and tile, ~0.1 us each, plus the fix-up's
+// launch. Measured, whole / split: [8192, 768 | 1536 | 3072] x [.., 768], 192 wide (128
+// tiles) 80.4 | 142.8 | 267 / 81.0 | 123.9 | 212 us, 256 wide (96) 98.5 | 175 | 328 / 84.6 |
+// 126 | 210; [15000, 1536] x [1536, 768], 192 wide (236) 186 / 223; [4096, 3072] x [3072, 768],
+// 192 wide (64) 277 / 117. 256 / 192 wide: N = 50272 over K = 768 5.71 / 5.99 ms; N = 3072
+// 345 / 364 us; N = 2304 (2.25 / 3 rounds) 286 / 273; N = 768 (192 / 256 tiles): K = 768
+// 99 / 94, K = 3072 367 / 349 us, K = 50272 5.82 / 5.63 ms.
 //
 // Chains. A sum over K rounds about 0.85 as much as on the f32 instruction
 // (split3.h), whose kernel splits every partly filled round: t 256 x 192 tiles short
@@ -1499,10 +1500,12 @@ SplitPlan gemm_split_plan(int64_t M, int64_t N, int64_t K, int64_t nb, int G, in
   const int64_t narrow = cdiv(M, VH_GEMMB_TM) * cdiv(N, VH_GEMMB_TN) * nb;
   const int64_t chains = std::max<int64_t>(1, std::min(cdiv(cdiv(G, narrow), ranges), K / 32));
   for (int64_t bn : {VH_GEMMB_TN_WIDE, VH_GEMMB_TN}) {
-    const double share = bn == VH_GEMMB_TN_WIDE ? 1.0 : 0.75, step = bn == VH_GEMMB_TN_WIDE ? 2.40 : 1.82;
+    const bool wide = bn == VH_GEMMB_TN_WIDE;
+    const double share = wide ? 1.0 : 0.75, step = wide ? 2.40 : 1.82;
     const int64_t tiles = cdiv(M, VH_GEMMB_TM) * cdiv(N, bn) * nb, rem = tiles % G;
-    const double whole =
-        nk * std::max(1.4 * share - step * (double)rem / G, 0.09 * share) + 9.0 * share * (double)(chains - 1);
+    const double f = (double)rem / G, alone = wide ? std::max(1.6, 0.77 + 1.63 * f) : std::max(1.3, 0.62 + 1.24 * f);
+    // Beyond the last round's share of full steps:
+    const double whole = 5.0 + nk * (alone - step * f) + 9.0 * share * (double)(chains - 1);
     const double split = 5.0 + 0.1 * share * (double)(G + rem);
     const double us = nk * step * (double)tiles / G + (rem ? std::min(whole, split) : 0.0);
     if (!best.bn || us < best.us) best = SplitPlan{bn, rem > 0 && whole < split ? (int)chains : 0, us};
