@@ -349,7 +349,7 @@ int vh_gemm_last_path(void);
 /* The name of the kernel that carried the calling thread's last vh_gemm (""
  * before any call, for an empty product, or on hipBLASLt): vh_gemms_* are the
  * persistent 256-row tiles on the bf16 instruction, vh_gemmb_* the same on the
- * f32 instruction, vh_gemmt_* the persistent walk of 64 x 64 tiles, vh_gemmp_* the
+ * f32 instruction, vh_gemmt_* the persistent walk of 64 x 64 tiles (_128: of 128 x 128), vh_gemmp_* the
  * walk over batched short-K products, vh_gemm_* the tiled kernel (_t64: its 64 x
  * 64 tiles). The string is the thread's own, valid until its next vh_gemm. */
 const char* vh_gemm_last_kernel(void);

@@ -2,6 +2,7 @@
 not cost: the tests of the other files name a kernel's sizes, this one holds the
 rule that picks it."""
 import ctypes
+import fnmatch
 
 import numpy as np
 import pytest
@@ -125,3 +126,26 @@ def test_chains_epilogue(vh, epi):
     assert vh.lib.vh_gemm_last_kernel().decode().startswith("vh_gemms")
     got = fetch(vh, C, (nb, M, N))
     assert np.all(np.abs(got - want) <= (K + 5) * 2.0 ** -24 * mag)
+
+
+@pytest.mark.parametrize("akc,bkc", [(True, True), (True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("M,N,K,want", [(256, 256, 65536, "vh_gemmt_??"), (300, 500, 16385, "vh_gemmt_??"),
+                                        (500, 520, 32769, "vh_gemmt_??_128"), (512, 768, 50272, "vh_gemmt_??_128"),
+                                        (2000, 1500, 17000, "vh_gemms_??_*")])
+def test_few_outputs_of_long_k(vh, M, N, K, want, akc, bkc):
+    """Few outputs over a K past 16384 walk the smaller tiles' K ranges in one launch;
+    more run on the 256-row tiles, a launch per range of K. The f32 instruction's error
+    bounds both, of the elements and of their sums over rows and columns (3: a drift
+    common to all would be 10 and more)."""
+    print("long k", M, N, K, akc, bkc, flush=True)
+    r = np.random.default_rng(K)
+    a = r.standard_normal((M, K)).astype(np.float32)
+    b = r.standard_normal((K, N)).astype(np.float32)
+    got, kernel = product(vh, a, b, akc, bkc)
+    assert fnmatch.fnmatch(kernel, want), kernel
+    f32 = product(vh, a, b, akc, bkc, engine=vh.GEMM_ENGINE_WIDE)[0]
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    d, e = got - ref, f32 - ref
+    assert np.linalg.norm(d) <= 1.05 * np.linalg.norm(e)
+    assert np.linalg.norm(d.sum(0)) <= 3 * np.linalg.norm(e.sum(0))
+    assert np.linalg.norm(d.sum(1)) <= 3 * np.linalg.norm(e.sum(1))

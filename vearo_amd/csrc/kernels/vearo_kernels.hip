@@ -245,9 +245,10 @@ K_GEMM(false, false, true, false, vh_gemm_m1_k1)
 K_GEMM(false, false, false, true, vh_gemm_m1_n4)
 K_GEMM(false, false, false, false, vh_gemm_m1_n1)
 // The 64 x 64 tiles walked by resident workgroups (products short of filling the
-// 256-row kernels).
-#define K_GEMMT(AK, BK, NAME) \
-  extern "C" __global__ void __launch_bounds__(256, 2) NAME(GemmArgs a) { gemm_tile_walk<AK, BK, 64>(a); }
+// 256-row kernels), and the 128 x 128 ones (_128: few outputs over a very long K).
+#define K_GEMMT(AK, BK, NAME)                                                                                     \
+  extern "C" __global__ void __launch_bounds__(256, 2) NAME(GemmArgs a) { gemm_tile_walk<AK, BK, 64>(a); }        \
+  extern "C" __global__ void __launch_bounds__(256, 2) NAME##_128(GemmArgs a) { gemm_tile_walk<AK, BK, 128>(a); }
 K_GEMMT(true, true, vh_gemmt_kk)
 K_GEMMT(true, false, vh_gemmt_kn)
 K_GEMMT(false, true, vh_gemmt_mk)

@@ -1550,12 +1550,14 @@ int gemm_split_k(const vh_gemm_desc* d, const GemmPlan& plan, int64_t lda, int64
   return rc;
 }
 
-// The 64 x 64 tiles walked by resident workgroups (three per CU).
+// The 64 x 64 (128 x 128) tiles walked by resident workgroups, three (two) per CU.
 int gemm_walk(const vh_gemm_desc* d, const GemmPlan& plan, bool akc, bool bkc, int64_t lda, int64_t ldb,
               hipStream_t s) {
   const int64_t nb = d->batch[0] * d->batch[1], tiles_m = cdiv(d->M, plan.tile), tiles_n = cdiv(d->N, plan.tile);
-  const int64_t grid = std::min<int64_t>(tiles_m * tiles_n * plan.ksplit * nb, 3 * std::max(g_rt.cu_count, 1));
-  const std::string name = std::string("vh_gemmt_") + (akc ? "k" : "m") + (bkc ? "k" : "n");
+  const int64_t grid =
+      std::min<int64_t>(tiles_m * tiles_n * plan.ksplit * nb, (plan.tile == 64 ? 3 : 2) * std::max(g_rt.cu_count, 1));
+  const std::string name =
+      std::string("vh_gemmt_") + (akc ? "k" : "m") + (bkc ? "k" : "n") + (plan.tile == 64 ? "" : "_128");
   if (plan.ksplit > 1) return gemm_split_k(d, plan, lda, ldb, name, grid, 1, s);
   GemmArgs g = gemm_args(d, lda, ldb, tiles_m, tiles_n);
   g.nbat = nb;
@@ -1600,19 +1602,25 @@ int gemm_split_range(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int
 int gemm_split(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t ldb, hipStream_t s, bool* taken) {
   *taken = false;
   if (!gemm_persistent_ok(d, lda, ldb)) return VH_OK;
+  const int64_t nb = d->batch[0] * d->batch[1], K = d->K, n = K > 16384 ? cdiv(K, 8192) : 1;
+  const int64_t kc = cdiv(cdiv(K, n), VH_GEMMS_TK) * VH_GEMMS_TK;
   // Below ~1e9 multiply-adds the 256-row tiles are too few or their pieces too many:
   // the 64 x 64 tiles where their estimate is less ([1000, 768] x [768, 768]: 36.7 us
-  // with its fix-up against 22.3; 5 us of launches are added to the other's). K <= 2
-  // never runs on the 256-row tiles: gemm.h has the f32 instruction there, which is
-  // more exact (2-norm error K = 1 2.53e-8 against the split's 3.44e-8, K = 2 3.11e-8
-  // against 3.36e-8, and 2.0 u against 2.8 u of sum |a b| at most; K = 3 3.60e-8 against
-  // 3.29e-8, 4 3.98e-8 against 3.24e-8).
-  const int64_t nb = d->batch[0] * d->batch[1];
-  const bool tiny = d->K <= 2;
-  if (d->K <= 16384 && (double)cdiv(d->M, 64) * (double)cdiv(d->N, 64) * (double)nb < 1e6) {
-    const GemmPlan tiled = gemm_plan(d->M, d->N, d->K, nb, nb == 1);
+  // with its fix-up against 22.3; 5 us of launches are added to the other's); the
+  // same, or 128 x 128 tiles, for few outputs over a K that runs in ranges ([256, 65536] x
+  // [65536, 256]: 470 -> 86 us, [512, 32768] x [32768, 512] 219 -> 115, [512, 50272] x
+  // [50272, 768] 374 -> 298), unless the estimates are close: it leaves out how full
+  // the walk's last round is ([1024, 20000] x [20000, 768], 528 items on 512 slots: 265
+  // us, estimated 210, against 215). K <= 2 never runs on the 256-row tiles: gemm.h has
+  // the f32 instruction there, which is more exact (2-norm error K = 1 2.53e-8 against
+  // the split's 3.44e-8, K = 2 3.11e-8 against 3.36e-8, and 2.0 u against 2.8 u of
+  // sum |a b| at most; K = 3 3.60e-8 against 3.29e-8, 4 3.98e-8 against 3.24e-8).
+  const bool tiny = K <= 2;
+  if ((double)cdiv(d->M, 64) * (double)cdiv(d->N, 64) * (double)nb < 1e6) {
+    const GemmPlan tiled = gemm_plan(d->M, d->N, K, nb, nb == 1);
     const int G = std::max(8, g_rt.cu_count / 8 * 8);
-    if (tiled.tile == 64 && (tiny || tiled.us < gemm_split_plan(d->M, d->N, d->K, nb, G).us + 5.0)) {
+    if ((tiled.tile == 64 || n > 1) &&
+        (tiny || tiled.us * (n > 1 ? 1.25 : 1.0) < (double)n * (gemm_split_plan(d->M, d->N, kc, nb, G, n).us + 5.0))) {
       VH_TRY(gemm_walk(d, tiled, akc, bkc, lda, ldb, s));
       *taken = true;
       g_gemm_path = VH_GEMM_PATH_PERSISTENT;
@@ -1620,8 +1628,6 @@ int gemm_split(const vh_gemm_desc* d, bool akc, bool bkc, int64_t lda, int64_t l
     }
   }
   if (tiny) return VH_OK;
-  const int64_t K = d->K, n = K > 16384 ? cdiv(K, 8192) : 1;
-  const int64_t kc = cdiv(cdiv(K, n), VH_GEMMS_TK) * VH_GEMMS_TK;
   for (int64_t k0 = 0; k0 < K; k0 += kc) {
     vh_gemm_desc t = *d;
     t.K = std::min(kc, K - k0);
