@@ -435,28 +435,40 @@ VH_DEV void GemmTile<A_KC, A_BUF, B_KC, B_BUF, T>::run(const GemmArgs& a, Lds& L
   for (int i = 0; i < NW; ++i)
 #pragma unroll
     for (int j = 0; j < NW; ++j) acc[i][j] *= S3_UNSCALE;
-  if (tiny || s3_nonfinite(acc)) {
-    // On the f32 instruction, straight from memory (see split3.h).
-#pragma unroll
-    for (int i = 0; i < NW; ++i)
-#pragma unroll
-      for (int j = 0; j < NW; ++j) acc[i][j] = vh_f32x16{};
+  // On the f32 instruction, straight from memory: all of a tiny product, or, a 32 x 32 tile
+  // at a time, the infinities and NaN of another (see split3.h). Rows past M (columns
+  // past N) and k past the range read as zero.
+  auto a_at = [&](int64_t m, int64_t k) { return m < a.M && k < ke ? A[A_KC ? m * a.lda + k : k * a.lda + m] : 0.0f; };
+  auto b_at = [&](int64_t n, int64_t k) { return n < a.N && k < ke ? B[B_KC ? n * a.ldb + k : k * a.ldb + n] : 0.0f; };
+  if (tiny) {
 #pragma nounroll
-    for (int64_t k0 = kb; k0 < ke; k0 += 2) {
-      const int64_t k = k0 + h;
-      float xa[NW], xb[NW];
+    for (int64_t k = kb; k < ke; k += 2) {
+      float x[NW], y[NW];
 #pragma unroll
       for (int i = 0; i < NW; ++i) {
-        const int64_t m = m0 + wm * (T / 2) + 32 * i + li, n = n0 + wn * (T / 2) + 32 * i + li;
-        xa[i] = m < a.M && k < ke ? A[A_KC ? m * a.lda + k : k * a.lda + m] : 0.0f;
-        xb[i] = n < a.N && k < ke ? B[B_KC ? n * a.ldb + k : k * a.ldb + n] : 0.0f;
+        x[i] = a_at(m0 + wm * (T / 2) + 32 * i + li, k + h);
+        y[i] = b_at(n0 + wn * (T / 2) + 32 * i + li, k + h);
       }
 #pragma unroll
       for (int i = 0; i < NW; ++i)
 #pragma unroll
-        for (int j = 0; j < NW; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[i], xb[j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < NW; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i], y[j], acc[i][j], 0, 0, 0);
     }
+  } else if (s3_nonfinite(acc)) {
+#pragma unroll
+    for (int i = 0; i < NW; ++i)
+#pragma unroll
+      for (int j = 0; j < NW; ++j) {
+        const int64_t mt = m0 + wm * (T / 2) + 32 * i, n = n0 + wn * (T / 2) + 32 * j + li;
+        const uint32_t bad = s3_nonfinite_regs(acc[i][j], a.M - mt - 4 * h, a.N - n);
+        if (__builtin_amdgcn_ballot_w64(bad != 0) == 0) continue;
+        vh_f32x16 t{};
+#pragma nounroll
+        for (int64_t k = kb; k < ke; k += 2)
+          t = __builtin_amdgcn_mfma_f32_32x32x2f32(a_at(mt + li, k + h), b_at(n, k + h), t, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = bad >> r & 1 ? t[r] : acc[i][j][r];
+      }
   }
 
   float* out = split ? a.ws + (int64_t)kr * a.M * a.N : C;

@@ -144,7 +144,6 @@ struct GbSplit {
 struct GbSeg {
   int m0, n0, kt0, kt1;
   int slot;  // -1: store C; else the workspace slot this partial piece goes to
-  bool more;  // gemm_split.h: a further chain of a tile whose C holds the ones before
   int64_t ao, bo, co, eo;
 };
 

@@ -107,13 +107,11 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
     GbSeg s;
     int u, kt0 = 0, kt1 = sp.nk;
     s.slot = -1;
-    s.more = false;
     if (j < ndp) {
       const int t = j / nch, c = j - t * nch;
       u = t * G + (t < sp.full ? local : xlo + g / 8);
       kt0 = sp.nk * c / nch;  // (the host keeps nk * nch below 2^31)
       kt1 = sp.nk * (c + 1) / nch;
-      s.more = c > 0;
     } else {
       const int p = j - ndp, t = t0 + p;  // (never with whole_tail)
       u = sp.full * G + t;
@@ -374,37 +372,42 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
     }
   };
   int s = 0;
-  // The block again on the f32 instruction, straight from memory, for a wave
-  // that met an infinity or a NaN (see split3.h): slow (~0.1 of the usual rate)
+  // What redo and epilogue read of the arguments they load again from the kernel's
+  // argument segment, behind a barrier to the compiler: held in scalar registers across
+  // the k loop, they would push its own into vector lanes.
+  auto args = []() {
+    auto p = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return (const GemmArgs*)p;
+  };
+  // The infinities and NaN of a wave's block again, a 32 x 32 tile at a time on the f32
+  // instruction straight from memory (see split3.h): slow (~0.1 of the usual rate)
   // and rare. Rows past M (columns past N) and k past K read as zero.
   auto redo = [&]() {
+    const GemmArgs& a = *args();
     const int64_t k1 = (int64_t)cur.kt1 * GS_TK < a.K ? (int64_t)cur.kt1 * GS_TK : a.K;
+    const float* A = a.A + cur.ao;
+    const float* B = a.B + cur.bo;
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
-      for (int jj = 0; jj < NB; ++jj) acc[i][jj] = vh_f32x16{};
-    const float* A = a.A + cur.ao;
-    const float* B = a.B + cur.bo;
-#pragma nounroll
-    for (int64_t k = (int64_t)cur.kt0 * GS_TK; k < k1; k += 2) {
-      const int64_t kk = k + h;
-      float fa2[WM], fb2[NB];
-#pragma unroll
-      for (int i = 0; i < WM; ++i) {
-        const int64_t m = cur.m0 + wm * WR + 32 * i + li;
-        fa2[i] = m < a.M && kk < k1 ? A[A_KC ? m * a.lda + kk : kk * a.lda + m] : 0.0f;
-      }
-#pragma unroll
       for (int jj = 0; jj < NB; ++jj) {
-        const int64_t n = cur.n0 + wn * WC + 32 * jj + li;
-        fb2[jj] = n < a.N && kk < k1 ? B[B_KC ? n * a.ldb + kk : kk * a.ldb + n] : 0.0f;
+        int l = li;
+        asm volatile("" : "+v"(l));  // (addresses formed here, as below)
+        const int64_t m0 = cur.m0 + wm * WR + 32 * i, m = m0 + l, n = cur.n0 + wn * WC + 32 * jj + l;
+        const uint32_t bad = s3_nonfinite_regs(acc[i][jj], a.M - m0 - 4 * h, a.N - n);
+        if (__builtin_amdgcn_ballot_w64(bad != 0) == 0) continue;
+        vh_f32x16 t{};
+#pragma nounroll
+        for (int64_t k = (int64_t)cur.kt0 * GS_TK; k < k1; k += 2) {
+          const int64_t kk = k + h;
+          const float x = m < a.M && kk < k1 ? A[A_KC ? m * a.lda + kk : kk * a.lda + m] : 0.0f;
+          const float y = n < a.N && kk < k1 ? B[B_KC ? n * a.ldb + kk : kk * a.ldb + n] : 0.0f;
+          t = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, t, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][jj][r] = bad >> r & 1 ? t[r] : acc[i][jj][r];
       }
-#pragma unroll
-      for (int jj = 0; jj < NB; ++jj)
-#pragma unroll
-        for (int i = 0; i < WM; ++i)
-          acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa2[i], fb2[jj], acc[i][jj], 0, 0, 0);
-    }
   };
   // The current segment's epilogue straight from the accumulators: register
   // r of a 32 x 32 tile holds row 8 (r / 4) + 4 h + r % 4, column li. A
@@ -414,6 +417,7 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
   // offsets where they are used instead of keeping them in registers across
   // the whole segment loop.
   auto epilogue = [&]() {
+    const GemmArgs& a = *args();
     const bool raw = cur.slot >= 0;
     int64_t ldo = raw ? BN : a.ldc;
     int lrow = wm * WR + 4 * h, lcol = wn * (BN / 2) + li;
@@ -435,8 +439,9 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
     using F = std::false_type;
     const bool inner = cur.m0 + GB_TM <= a.M && cur.n0 + BN <= a.N;
     float* const Cb = a.C + cur.co;
-    const float* const Eb = a.E && !cur.more ? a.E + cur.eo : nullptr;
-    const bool accumulate = a.accumulate || cur.more;
+    const bool more = cur.kt0 > 0;  // a further chain: C holds the ones before, E and the old C among them
+    const float* const Eb = a.E && !more ? a.E + cur.eo : nullptr;
+    const bool accumulate = a.accumulate || more;
     if (inner && !Eb && !accumulate) {
       float* base = Cb + (cur.m0 + lrow) * ldo + cur.n0 + lcol;
 #pragma unroll

@@ -30,7 +30,9 @@
 // a finite value that is infinite as bf16 once scaled (above 5.2e33); sums overflow
 // from 7.9e28. All of these give an infinity or a NaN in every output they reach,
 // so an accumulator that comes out finite is right, and a wave that finds one that
-// is not recomputes its block with the f32 instruction, which has IEEE's answer.
+// is not recomputes its 32 x 32 tile on the f32 instruction, which has IEEE's answer,
+// and takes from there the elements that were not finite, and only those: what one
+// output is does not depend on the values of another's row or column.
 #pragma once
 #include "common.h"
 
@@ -95,6 +97,22 @@ VH_DEV vh_f32x16 s3_mfma(const vh_u4& a, const vh_u4& b, const vh_f32x16& acc) {
 #define S3_UNSCALE 2.3283064365386963e-10f  // on their products' sum (2^-32)
 #define S3_PA(T) ((T) == 0 ? 2 : (T) == 1 ? 0 : (T) == 2 ? 1 : (T) == 3 ? 1 : 0)  // A's part in product T
 #define S3_PB(T) ((T) == 0 ? 0 : (T) == 1 ? 2 : (T) == 2 ? 1 : (T) == 4 ? 1 : 0)  // B's part
+
+// The registers of a 32 x 32 accumulator tile (bit r: register r) that hold an
+// infinity or a NaN in a row below mlim and a column below nlim, both counted from the
+// lane's first row and its column. One register after the other: sixteen lane masks at
+// once would take the scalar registers that the callers' loops keep their state in.
+VH_DEV uint32_t s3_nonfinite_regs(const vh_f32x16& acc, int64_t mlim, int64_t nlim) {
+  const int ml = nlim <= 0 || mlim < 0 ? 0 : mlim < 32 ? (int)mlim : 32;
+  uint32_t bad = 0;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const uint32_t below = (uint32_t)(8 * (r >> 2) + (r & 3) - ml) >> 31;
+    bad |= __builtin_fabsf(acc[r]) < __builtin_inff() ? 0u : below << r;
+    asm volatile("" : "+v"(bad));
+  }
+  return bad;
+}
 
 // Whether any of a wave's accumulators is an infinity or a NaN (x * 0 is then NaN).
 template <int I, int J>
