@@ -244,13 +244,20 @@ struct vb_gpt {
       VB(vh_gemm(&d, nullptr));
     }
     // dW = dlogits^T lnf straight into the gradient's [Vp, D] layout: A is
-    // dlogits read row-contiguous (m-contiguous), B is lnf. It stays on the f32
-    // instruction (8.85 ms; the split kernel runs it in 5.6): in the rows of
-    // frequent tokens a sum of ~16384 terms holds a few large ones (-1 / R x per
-    // hit) and many of 1e-5 that size, which one rounding per k loses under the
-    // sum and the split's rounding per eight products does not -- 7.7e-5 against
-    // 5.4e-6 of the gradient's norm from the 64-bit one, so the two kernels'
-    // results differ by 6e-5, more than this gradient may change by.
+    // dlogits read row-contiguous (m-contiguous), B is lnf. Long sums over large
+    // vocabularies stay on the f32 instruction (at R = 16384, V = 50257 8.85 ms; the
+    // split kernel runs it in 5.6): in the rows of frequent tokens a sum holds a few
+    // terms of hits / R and many of 1 / (V R), which the f32 chain loses under it, the
+    // more the larger V R (they fall below half its last place from ~3e8), and the
+    // split's rounding per eight products does not. Measured, this gradient's error
+    // against 64-bit sums, f32 / split, and their difference: V = 50257, R = 1024 5.0e-7 /
+    // 3.2e-7, 5.7e-7; 4096 3.8e-6 / 5.6e-7, 3.6e-6; 8192 3.2e-5 / 2.2e-6, 3.0e-5; 16384
+    // 7.3e-5 / 5.2e-6, 6.8e-5. The split's is the better one at every size, but the
+    // step's gradients are held to 2e-5 of what they have been (perf/cases.py), so it
+    // carries the product where the two differ by less: over 11 pairs of R and V with 5
+    // batches each, by 8.9e-6 at most up to V R = 2^27, by up to 3.5e-5 at 2e8. (The
+    // BackendOps step, backend/dropin_gpt.cpp, runs the split at every size.)
+    const bool f32_dw = engine == VH_GEMM_ENGINE_DEFAULT && Vp * R >= (int64_t(1) << 27);
     {
       vh_gemm_desc d{};
       d.M = Vp;
@@ -266,7 +273,7 @@ struct vb_gpt {
       d.c_sm = D;
       d.batch[0] = d.batch[1] = 1;
       d.alpha = 1.0f;
-      d.engine = engine == VH_GEMM_ENGINE_DEFAULT ? VH_GEMM_ENGINE_WIDE : engine;
+      d.engine = f32_dw ? VH_GEMM_ENGINE_WIDE : engine;
       VB(vh_gemm(&d, nullptr));
     }
     VB(vh_layernorm_bwd(h2, p(18), dlnf, dh, gr(18), gr(19), R, D, kEps, nullptr, 0, nullptr));
