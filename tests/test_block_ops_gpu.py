@@ -63,9 +63,9 @@ def test_matmul_reference_kats(vh):
     assert run_matmul(vh, a, b.T, b_view="T").tolist() == O.matmul(a, b.T).tolist()
 
 
-# N <= 64 takes the 128 x 64 tile; with 128-bit loads its k tiles run two
-# steps ahead in pairs: (128, 32, 64) one step, (256, 96, 64) and
-# (384, 160, 64) odd step counts, (200, 288, 60) edge tiles with the checked loop.
+# These sizes take the tiled kernel's 64 x 64 tiles, whose 32-wide k tiles are loaded two
+# ahead in pairs: (128, 32, 64) one k tile, (256, 96, 64) and (384, 160, 64) odd counts,
+# (200, 288, 60) edge tiles.
 @pytest.mark.parametrize("M,K,N", [(1, 1, 1), (5, 7, 3), (128, 32, 128), (129, 33, 131),
                                    (300, 768, 200), (64, 1000, 96), (257, 64, 513),
                                    (300, 200, 64), (257, 96, 33), (1024, 1024, 64),
@@ -552,11 +552,10 @@ def test_gemm_split_k(vh, M, N, K):
     np.testing.assert_array_equal(fetch(vh, C3, (M, N)), got)
 
 
-# The persistent 256 x 192-tile kernel at the block step's shapes (fewer rows
-# where the full product would keep the oracle busy): every layout pair, tile
-# edges in M and N, a stream-K last round (tiles mod CUs != 0), a ragged K
-# (50260 = 1570 x 32 + 20: the tiled kernel adds the tail), and the Linear
-# epilogues (bias, bias + residual accumulation, alpha). A is N(0,1) times
+# The persistent kernels (256-row tiles, or the walk of smaller ones) at the block
+# step's shapes (fewer rows where the full product would keep the oracle busy):
+# every layout pair, tile edges in M and N, last rounds split and left whole, a ragged
+# K, and the Linear epilogues (bias, bias + residual accumulation, alpha). A is N(0,1) times
 # a_scale: lm_head dx's A is dlogits, whose entries are ~1e-4 (softmax over
 # 50257 classes, divided by the row count), so a 50260-term row sum of it
 # stays far from cancellation; the plain cases also meet the f32 error bound
@@ -640,11 +639,9 @@ def test_gemm_persistent_block_shapes(vh, case):
 
 
 def test_gemm_persistent_few_k_tiles_after_workspace_reuse(vh):
-    """Stream-K with fewer k tiles than workgroups leaves some workgroups an
-    empty run inside a split tile; the fix-up must skip their workspace slots,
-    which hold whatever an earlier product left there. A product with many
-    partial pieces first fills the (reused) workspace, then products with
-    102 and 120 k tiles in their stream-K round run against the oracle."""
+    """Small products after one whose partial pieces fill the (reused) workspace.
+    (Empty runs of the split round, whose slots the fix-up must skip, need more
+    tiles: test_gemm_kernels_gpu.py.)"""
     r = np.random.default_rng(21)
     def prod(M, N, K):
         a = r.standard_normal((M, K), dtype=np.float32)
@@ -673,11 +670,10 @@ BATCHED_PERSISTENT_CASES = [
 @pytest.mark.parametrize("case", BATCHED_PERSISTENT_CASES, ids=[c[0] for c in BATCHED_PERSISTENT_CASES])
 def test_gemm_persistent_batched(vh, case):
     """Batched dense products with k loops of 512 and more on the persistent
-    kernel: the tile list runs over every batch (tile-major within a batch),
-    each segment offsets A, B, C and the addend by its batch's strides, and a
-    batch's k-contiguous tail past the whole k tiles goes through the tiled
-    kernel. Against the oracle's batched matmul and float64, and the same bits
-    on a second call."""
+    walk of 64 x 64 tiles: the tile list runs over every batch, each tile offsets A,
+    B, C and the addend by its batch's strides. Against the oracle's batched matmul
+    and float64, and the same bits on a second call. (Batches on the 256-row
+    kernel: test_gemm_kernels_gpu.py.)"""
     name, (B0, B1), M, N, K, akc, bkc, shared, epi = case
     print("persistent batched", name, flush=True)
     r = np.random.default_rng(M + N + K)

@@ -1,9 +1,11 @@
-"""The split persistent product (kernels/gemm_split.h): f32 operands as three bf16
-parts each, six part products on the bf16 matrix instruction. Sizes where its
-tiles, k tail, last round and k ranges can go wrong, every operand layout, against
-float64; infinities, NaN, values whose bf16 rounding overflows and subnormals, which
-the split cannot carry and the kernel recomputes; and its error against the f32
-instruction's.
+"""Products as three-part splits (kernels/split3.h): f32 operands as three bf16
+parts each, six part products on the bf16 matrix instruction. Every operand layout,
+edges and k tails against float64; infinities, NaN, values whose bf16 rounding
+overflows and subnormals, which the split cannot carry and the kernels recompute;
+and the error against the f32 instruction's. Of the large sizes below, the
+256-row kernel (kernels/gemm_split.h) runs [4097, 32] x [32, 3071] and K = 16384 of the
+error test, the walk of 64 x 64 tiles (kernels/gemm.h) the others; the 256-row kernel's
+own sizes are in test_gemm_kernels_gpu.py, by the kernel's name.
 
 Bound: a sum of K products in f32 is within K u sum |a||b| of the exact one in any
 order (u = 2^-24); the split's 12 roundings per 16 k are fewer than K, and the part
@@ -40,11 +42,11 @@ def product(vh, a, b, akc, bkc, off=0, **kw):
 LAYOUTS = [(True, True), (True, False), (False, True), (False, False)]
 #   M, N, K, floats off 16-byte alignment
 SIZES = [
-    (256, 192, 1366, 0),    # one tile, k tail of 6, split over all workgroups
-    (257, 193, 1361, 1),    # one row and one column past a tile, k tail of 1
+    (256, 192, 1366, 0),    # whole 64 x 64 tiles, k tail of 22
+    (257, 193, 1361, 1),    # one row and one column past a tile, k tail of 17
     (1000, 777, 1007, 3),   # ragged, k tail of 15
-    (4097, 3071, 32, 0),    # 17 x 12 tiles of two k tiles, last round left whole
-    (300, 500, 16385, 0),   # past the single-chain limit: three k ranges, the last ragged
+    (4097, 3071, 32, 0),    # 256-row tiles of two k tiles, the round left whole
+    (300, 500, 16385, 0),   # past the 256-row kernel's single-chain limit
 ]
 
 
@@ -145,7 +147,8 @@ def test_split_product_error_is_no_larger(vh, K, one_signed):
 # ------------------------------------------------ the tiled kernel (kernels/gemm.h) --
 
 #   M, N, K, floats off alignment: K <= 8 on the f32 instruction, then edges of its 64 x
-#   64 and 128 x 128 tiles and of its 32-wide k tiles, one and several of each.
+#   64 tiles and of its 32-wide k tiles, one and several of each (its 128 x 128 tiles:
+#   test_gemm_kernels_gpu.py).
 TILE_SIZES = [(64, 64, 1, 0), (65, 63, 8, 1), (63, 65, 9, 0), (1, 200, 33, 3), (200, 1, 31, 0), (129, 127, 95, 2),
               (64, 128, 32, 0), (700, 130, 65, 1), (255, 300, 2049, 1), (2048, 191, 100, 0)]
 

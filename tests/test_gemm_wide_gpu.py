@@ -1,10 +1,9 @@
-"""The persistent GEMM's wide tile (256 x 256, kernels/gemm_big.h). vh_gemm
-picks it for long k loops (K >= 8192 in whole k tiles) over a row-contiguous
-B with at least one full round of wide tiles -- the block step's lm_head dW
-([50260, 768] = dlogits^T ln_f) -- and the WIDE engine forces it wherever the
-persistent kernel runs, so these products stay small enough for the CPU
-oracle. Every operand layout, edges in M and N, a k tail left to the tiled
-kernel, bias / accumulate / alpha epilogues, operands only 4-byte aligned, and
+"""The f32-instruction persistent GEMM's 256 x 256 tile (kernels/gemm_big.h), which the
+WIDE engine runs on every large dense product of 256 columns and more (its 256 x 192
+tile below: test_gemm_kernels_gpu.py); the block step's lm_head dW ([50260, 768] =
+dlogits^T ln_f) takes it for long sums over large vocabularies. The products stay
+small enough for the CPU oracle. Every operand layout, edges in M and N, a k tail left to
+the tiled kernel, bias / accumulate / alpha epilogues, operands only 4-byte aligned, and
 the stream-K round with its fix-up (fixed order: the same bits on a second
 call); against the oracle, float64 and the f32 error bound of a K-term sum."""
 import ctypes
