@@ -298,21 +298,26 @@ size_t vh_sum_rows_scratch_bytes(int64_t rows, int64_t C);
 
 /* vh_gemm_desc.engine: which kernels carry the product. The default is this
  * library's own matrix-core kernels, chosen by shape (large dense products: the
- * persistent 256-row-tile kernel, whose f32 products run as exact three-part
- * bf16 splits; everything else: the tiled kernel, split along K where the output
- * alone cannot fill the chip). TILED forces the tiled kernel (tests of its
- * split-K path); LIBRARY hands the dense unbatched products hipBLASLt supports to
- * it (an A/B reference for benchmarks) and runs the rest as DEFAULT; WIDE is
- * DEFAULT with the large dense products on the f32 matrix instruction (the
- * persistent kernel's 256 x 256 tile): every k rounds into the f32 sum on its own,
- * in one fixed order. No counterpart in the reference. */
+ * persistent 256-row-tile kernel, or a persistent walk of smaller tiles; everything
+ * else: the tiled kernel, split along K where the output alone cannot fill the
+ * chip). All run f32 products as three-part bf16 splits, but those of K <= 2 (K <= 8 on
+ * the smaller tiles), which stay on the f32 matrix instruction. TILED forces the
+ * tiled kernel (tests of its split-K path); LIBRARY hands the dense unbatched
+ * products hipBLASLt supports to it (an A/B reference for benchmarks) and runs the
+ * rest as DEFAULT; WIDE is DEFAULT with the large dense products (M >= 256, N >= 192, 2^26
+ * multiply-adds; smaller ones run as DEFAULT) on the f32 matrix instruction, on
+ * 256 x 256 tiles (256 x 192 below 256 columns): every k rounds into the f32 sum on its
+ * own, in one fixed order. Infinities, NaN and sums past the splits' range come
+ * out as f32 arithmetic has them, and leave the bits of other outputs as they
+ * are; a product full of them runs at about a tenth of its rate. No counterpart in
+ * the reference. */
 #define VH_GEMM_ENGINE_DEFAULT 0
 #define VH_GEMM_ENGINE_TILED 1
 #define VH_GEMM_ENGINE_LIBRARY 2
 #define VH_GEMM_ENGINE_WIDE 3
 
 /* C[m, n] = (C[m, n] +) alpha * sum_k A[m, k] B[k, n] (+ E[m, n]) over two batch
- * dims, on the f32 matrix cores. The epilogue order is v = acc*alpha;
+ * dims, f32 in and out, on the matrix cores. The epilogue order is v = acc*alpha;
  * v = v + E; v = C + v, i.e. the separate scale / mask / bias-add / gradient
  * accumulation ops the reference applies after its matmul. */
 typedef struct vh_gemm_desc {

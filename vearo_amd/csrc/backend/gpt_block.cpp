@@ -221,8 +221,9 @@ struct vb_gpt {
     // dlogits came with the forward (forward(true)). lm_head (rank-2 input, no bias), over the padded vocabulary: the zero
     // columns of dlogits meet the zero rows after the weight.
     // dx = dlogits W reads W through a transposed copy: both operands are then
-    // k-contiguous, which the large-product kernel runs faster than W's
-    // row-contiguous form (8.6 against 8.8 ms; the 154 MB copy costs ~90 us).
+    // k-contiguous. The split kernel runs that form in 5.69-5.72 ms and W's
+    // row-contiguous one in 5.71-5.77, so the copy (59 us) gains it nothing; the f32
+    // kernel ran them in 8.6 and 8.8, the library's in the first.
     {
       const vh_layout wl{2, 0, {D, Vp}, {1, D}};
       VB(vh_strided_copy(p(20), &wl, wT, nullptr));

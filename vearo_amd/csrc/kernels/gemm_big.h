@@ -1,8 +1,9 @@
-// gemm_big.h -- f32 matrix multiply for the large dense products (the lm_head
-// and Linear layers of the GPT block step) on the gfx950 matrix cores.
+// gemm_big.h -- f32 matrix multiply for large dense products on the f32 matrix
+// instruction of gfx950: the WIDE engine, and with it the lm_head weight gradient of
+// long sums in the GPT block step (gemm_split.h carries the others).
 //
 // Same semantics and epilogue as gemm.h (C = alpha A B (+ E) (+ C), each
-// operand k-contiguous or row-contiguous), for unbatched, non-causal products
+// operand k-contiguous or row-contiguous), for non-causal products
 // whose operands allow 128-bit loads and 32-bit tile offsets, and whose
 // k-contiguous operands have K % 32 == 0 (the host checks; it runs a ragged
 // k tail as a second, accumulating product, and everything else on gemm.h).
