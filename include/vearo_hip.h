@@ -309,7 +309,7 @@ size_t vh_sum_rows_scratch_bytes(int64_t rows, int64_t C);
  * 256 x 256 tiles (256 x 192 below 256 columns): every k rounds into the f32 sum on its
  * own, in one fixed order. Infinities, NaN and sums past the splits' range come
  * out as f32 arithmetic has them, and leave the bits of other outputs as they
- * are; a product full of them runs at about a tenth of its rate. No counterpart in
+ * are; a product full of them takes about five times as long. No counterpart in
  * the reference. */
 #define VH_GEMM_ENGINE_DEFAULT 0
 #define VH_GEMM_ENGINE_TILED 1

@@ -386,13 +386,14 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
     return (const GemmArgs*)p;
   };
   // The infinities and NaN of a wave's block again, a 32 x 32 tile at a time on the f32
-  // instruction straight from memory (see split3.h): slow (~0.1 of the usual rate)
-  // and rare. Rows past M (columns past N) and k past K read as zero.
+  // instruction straight from memory (see split3.h). [16384, 768] x [768, 3072] full of
+  // NaN takes 1.36 ms (operands k-contiguous) or 1.87 (row-contiguous) against 0.34 of
+  // numbers, with one infinity 0.45 or 0.54. Two or more tiles at a time would share
+  // their loads (1.13 and 1.27), but take registers from the usual path (0.34 -> 0.35).
+  // A row past M (column past N) reads the last one's: none of its outputs is replaced.
   auto redo = [&]() {
     const GemmArgs& a = *args();
     const int64_t k1 = (int64_t)cur.kt1 * GS_TK < a.K ? (int64_t)cur.kt1 * GS_TK : a.K;
-    const float* A = a.A + cur.ao;
-    const float* B = a.B + cur.bo;
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -402,13 +403,32 @@ VH_DEV void gemm_split_impl(const GemmArgs& a) {
         const int64_t m0 = cur.m0 + wm * WR + 32 * i, m = m0 + l, n = cur.n0 + wn * WC + 32 * jj + l;
         const uint32_t bad = s3_nonfinite_regs(acc[i][jj], a.M - m0 - 4 * h, a.N - n);
         if (__builtin_amdgcn_ballot_w64(bad != 0) == 0) continue;
+        // Lane half h takes k + 4 h .. k + 4 h + 3 of every eight k, one load where they lie
+        // together.
+        const int64_t k0 = (int64_t)cur.kt0 * GS_TK + 4 * h;
+        const int64_t mc = m < a.M ? m : a.M - 1, nc = n < a.N ? n : a.N - 1;
+        const float* pa = a.A + cur.ao + (A_KC ? mc * a.lda + k0 : k0 * a.lda + mc);
+        const float* pb = a.B + cur.bo + (B_KC ? nc * a.ldb + k0 : k0 * a.ldb + nc);
+        auto load = [&](auto kc, const float* p, int64_t ld, int left, float (&v)[4]) {
+          if (decltype(kc)::value && left >= 8) {
+            const s3_f4u q = *reinterpret_cast<const s3_f4u*>(p);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = q[u];
+          } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = 4 * h + u < left ? p[decltype(kc)::value ? u : u * ld] : 0.0f;
+          }
+        };
         vh_f32x16 t{};
 #pragma nounroll
-        for (int64_t k = (int64_t)cur.kt0 * GS_TK; k < k1; k += 2) {
-          const int64_t kk = k + h;
-          const float x = m < a.M && kk < k1 ? A[A_KC ? m * a.lda + kk : kk * a.lda + m] : 0.0f;
-          const float y = n < a.N && kk < k1 ? B[B_KC ? n * a.ldb + kk : kk * a.ldb + n] : 0.0f;
-          t = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, t, 0, 0, 0);
+        for (int left = (int)(k1 - (int64_t)cur.kt0 * GS_TK); left > 0; left -= 8) {
+          float x[4], y[4];
+          load(akc, pa, a.lda, left, x);
+          load(bkc, pb, a.ldb, left, y);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) t = __builtin_amdgcn_mfma_f32_32x32x2f32(x[u], y[u], t, 0, 0, 0);
+          pa += A_KC ? 8 : 8 * a.lda;
+          pb += B_KC ? 8 : 8 * a.ldb;
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][jj][r] = bad >> r & 1 ? t[r] : acc[i][jj][r];

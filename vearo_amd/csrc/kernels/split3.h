@@ -41,6 +41,7 @@ typedef __bf16 vh_bf2 __attribute__((ext_vector_type(2)));
 typedef __bf16 vh_bf8 __attribute__((ext_vector_type(8)));
 typedef float vh_f2 __attribute__((ext_vector_type(2)));
 typedef uint32_t vh_u4 __attribute__((ext_vector_type(4)));
+typedef float s3_f4u __attribute__((ext_vector_type(4), aligned(4)));  // at any float's address
 
 // Two values -> their three parts, each pair packed in one register (x0 low):
 // three v_cvt_pk_bf16_f32, four subtractions and four half extractions.
